@@ -247,7 +247,7 @@ wl_status wl_run_chain(wl_ctx* ctx, uint32_t first_layer, uint32_t n_layers, flo
  * partly overlap them; all three 16-byte aligned). Each token is routed exactly as wl_run_moe routes
  * it (same ids); tokens are then
  * grouped by expert (stable, (token, slot) order) and every selected expert's
- * weights are streamed once per 32 of its tokens; the per-token combine sums
+ * weights are read once per pass of up to 80 of its tokens (down: 64); the per-token combine sums
  * the slots in slot order, then the shared expert (the reference's pass 3).
  * A layer with every expert bound runs with no host round trip; a layer with
  * none bound fetches its routed set through the context's expert source (see

@@ -1,0 +1,842 @@
+// batched_gemm.h — the expert GEMMs of the batched layer (included by
+// moe_batched.hip, inside namespace wl).
+//
+// Every work-group is eight waves with a whole CU (LDS), two per SIMD, so that
+// one wave's matrix instructions run while the other is held at a load: issuing
+// the loads takes about as long as the matrix instructions (measured at 64-token
+// passes with one wave per SIMD and twice the tiles per wave: a step of 2560
+// cycles of MFMA took 4576, the loads adding 112 cycles each). A pipeline runs
+// units of one form (a token pass of NB row blocks of 16 tokens times a block of
+// weight rows, in nst steps of K): the bf16 shared expert (SharedK), then the
+// routed passes from five row blocks down to one (QWide, QNarrow). A work-group
+// walks its units u = blockIdx.x + G i of each pipeline. Activations arrive in
+// LDS by DMA (buffer_load ... lds), weights in registers. The weights are the
+// matrix instructions' A operand (its rows), the tokens its columns: a lane then
+// holds four consecutive outputs of one token, stored as 16 bytes.
+#pragma once
+
+constexpr uint32_t kSlotB = 48u << 10;
+constexpr uint32_t kOOBV = 0x80000000u;  // a lane offset past every array (they stay below 2 GB)
+// Three slots of activations, separate LDS objects so that the compiler's own
+// waits for DMA-written LDS stay per slot.
+__shared__ __align__(16) uint8_t g_slot0[kSlotB];
+__shared__ __align__(16) uint8_t g_slot1[kSlotB];
+__shared__ __align__(16) uint8_t g_slot2[kSlotB];
+template <int S>
+WL_DEV uint8_t* slot() {
+    return S == 0 ? g_slot0 : S == 1 ? g_slot1 : g_slot2;
+}
+template <int S>
+WL_DEV void dma16(rsrc_t rs, uint32_t lds, uint32_t voff, uint32_t soff) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(slot<S>() + lds), 16u, voff,
+                                             soff, 0, 0);
+}
+// s_waitcnt vmcnt(N) (expcnt, lgkmcnt not waited on), barrier.
+template <uint32_t N>
+WL_DEV void step_barrier() {
+    static_assert(N < 64u, "vmcnt is 6 bits");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt((N & 15u) | ((N >> 4) << 14) | 0x0F70u);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+// Between two pipelines of one kernel: every load and DMA of the first has
+// landed and every wave is done with its slots.
+WL_DEV void pipeline_drain() { step_barrier<0>(); }
+
+// A unit: a token pass (of the batch, or an expert's) and its block of weight
+// rows.
+struct UnitInfo {
+    bool live;
+    uint32_t e, part, nt, row0;
+};
+
+// ---- pipeline ------------------------------------------------------------------------
+// Position of a stream in the units' steps: my unit i, its step s.
+struct Cursor {
+    uint32_t i, s;
+};
+WL_DEV bool advance(Cursor& c, uint32_t nst) {
+    if (++c.s < nst) return false;
+    c.s = 0;
+    c.i++;
+    return true;
+}
+// The steps of a work-group's units form one flat sequence z. A pipeline has one
+// form of unit, so that every value keeps its registers through the loop (with
+// forms chosen per unit the compiler moved the loads in flight between registers
+// at the units' ends, which waits for them). The loads run two steps ahead
+// of the compute, through the units' ends. Step z: this wave's loads of the step,
+// issued two steps ago, have landed ("at most the loads of one step
+// outstanding": they complete in issue order) and the waves have met, so every
+// wave's activations are there and every wave is done with step z - 1, whose slot
+// and registers take the loads of step z + 2; these go out evenly between the
+// matrix instructions of step z (all at its start: 7 to 18 % slower per call). The loop runs whole rounds
+// of three steps; the loads of the steps past the last unit are out of range
+// (zeros) and what they compute is not stored.
+template <int S, class Kn>
+WL_DEV void unit_step(Kn& k, typename Kn::AS& A, typename Kn::WB& cur, typename Kn::WB& nxt) {
+    constexpr uint32_t L = Kn::kDmas + Kn::kLoads;
+    constexpr int SN = (S + 2) % 3;
+    step_barrier<L>();
+    if (advance(k.cn, k.nst)) k.bind(k.cn.i, A);
+    const uint32_t sn = k.cn.s;
+    // called n times over a step (it = 0 .. n - 1)
+    auto next = [&](uint32_t it, uint32_t n) {
+#pragma unroll
+        for (uint32_t j = 0; j < L; j++) {
+            if (j * n / L != it) continue;
+            if (j < Kn::kDmas) k.template dma<SN>(A, sn, j);
+            else k.load(sn, nxt, j - Kn::kDmas);
+        }
+    };
+    __builtin_amdgcn_sched_barrier(0);
+    k.comp(k.cc.s, slot<S>(), cur, next);
+    if (advance(k.cc, k.nst)) {
+        if (k.cc.i <= k.nu) k.finish();
+        k.begin(k.cc.i);
+    }
+}
+template <class Kn>
+WL_DEV void run_units(Kn& k) {
+    if (k.nu == 0u) return;
+    const uint32_t Z = k.nu * k.nst;
+    typename Kn::AS A;
+    typename Kn::WB B0, B1, B2;
+    k.cn = k.cc = Cursor{0u, 0u};
+    k.begin(0u);
+    k.bind(0u, A);
+#pragma unroll
+    for (uint32_t j = 0; j < Kn::kDmas; j++) k.template dma<0>(A, 0u, j);
+#pragma unroll
+    for (uint32_t j = 0; j < Kn::kLoads; j++) k.load(0u, B0, j);
+    if (advance(k.cn, k.nst)) k.bind(k.cn.i, A);
+#pragma unroll
+    for (uint32_t j = 0; j < Kn::kDmas; j++) k.template dma<1>(A, k.cn.s, j);
+#pragma unroll
+    for (uint32_t j = 0; j < Kn::kLoads; j++) k.load(k.cn.s, B1, j);
+#pragma unroll 1
+    for (uint32_t z = 0; z < Z; z += 3u) {
+        unit_step<0>(k, A, B0, B2);
+        unit_step<1>(k, A, B1, B0);
+        unit_step<2>(k, A, B2, B1);
+    }
+}
+
+// ---- outputs ---------------------------------------------------------------------------
+// The epilogues pass the lane through opaque_lane, so the compiler cannot hoist
+// their per-row addresses out of the step loop.
+WL_DEV uint32_t opaque_lane() {
+    uint32_t l = threadIdx.x & 63u;
+    asm volatile("" : "+v"(l));
+    return l;
+}
+// SwiGLU of two gate/up tiles (rows 0-7 gate, 8-15 the matching up rows; lane
+// (n, g) holds rows 4g .. 4g + 3 of token n): one swap per value brings the gate
+// values of both tiles together and their up values, so lane (n, g) gets columns
+// 4 (g % 2) .. +4 of tile g / 2 for token n.
+WL_DEV f32x4 swiglu_pair(const f32x4& a, const f32x4& b) {
+    f32x4 r;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) {
+        uint32_t gt, up;
+        swap32(__float_as_uint(a[i]), __float_as_uint(b[i]), gt, up);
+        r[i] = silu_mul(__uint_as_float(gt), __uint_as_float(up));
+    }
+    return r;
+}
+
+// ---- shared expert (bf16) ----------------------------------------------------------------
+// Three bf16 pieces of each activation (x = p0 + p1 + p2 to f32 precision)
+// through v_mfma_f32_16x16x32_bf16; the first piece and the other two sum in
+// accumulators of their own, and with NT = 1 the first piece's are added to the
+// sums at every step (a long chain of matrix instructions rounds more often). Unit: a pass of the batch (its tokens split evenly
+// over cdiv(T, 64) passes, NB row blocks) x 8 waves x NT tiles. UP: tiles of 8
+// gate and 8 up rows (native sgu chunks: lane (n, g) row n, columns [32 kt + 8
+// g, +8)), K = H, SwiGLU values as pieces to smid3. Otherwise tiles of 16 output
+// rows (native sdn: 16 bytes = columns [8T, +8) of a row, lane (n, g) tile 4 kt +
+// g of row n), K = SI, f32 rows to shout. A step is 128 columns. NT = 1: small
+// batches, more units; NT = 2: a fragment feeds two tiles.
+//
+// Slot: row R = 64 pc + m (token m, piece pc) of 256 bytes, its 16-byte group p
+// holding columns [k0 + 8 (p ^ (R & 15)), +8), so that the 16 rows a fragment
+// reads at one column fall in 16 different bank groups. A DMA of wave v writes rows
+// 64 pc + 32 j + r0, r0 = 4 v + (lane >> 4) < 32, of piece pc (j = 0, 1).
+struct AStreamS {
+    rsrc_t rs;
+    uint32_t base[2], kd2;  // lane byte offsets of the tokens r0 + 32 j (kOOBV: none), bytes per piece row
+};
+template <bool UP, uint32_t NT, uint32_t NB>
+struct SharedK {
+    using AS = AStreamS;
+    struct WB {
+        u32x4 w[4 * NT];
+    };
+    static constexpr uint32_t kLoads = 4 * NT, kRB2 = (NB + 1) / 2, kDmas = 3 * kRB2;
+    const DecodeArgs& a;
+    const BatchArgs& b;
+    uint32_t H, SI, nkt, parts, npass, nst, nu, v, n, g;
+    Cursor cn, cc;  // positions of the loads and of the compute
+    // weight stream: the block, kept as a pointer and a size (a buffer resource
+    // held in a struct has gone through scratch, its loads per-lane loops)
+    const uint8_t* wbase;
+    uint32_t wbytes, wpart, vw[UP ? 1 : NT], lob;
+    UnitInfo cu;
+    static constexpr bool kSum = NT == 1u;
+    f32x4 acc[NT][NB][2], sum[kSum ? NT : 1][kSum ? NB : 1];
+
+    WL_MEM UnitInfo unit(uint32_t i) const {
+        UnitInfo x{false, 0u, 0u, 0u, 0u};
+        if (i >= nu) return x;
+        const PassPart jp = pass_part(blockIdx.x + gridDim.x * i, parts, npass);
+        x.live = true;
+        x.part = jp.part;
+        const uint32_t q = b.T / npass, r = b.T % npass;
+        x.row0 = jp.j * q + min(jp.j, r);
+        x.nt = q + (jp.j < r ? 1u : 0u);
+        return x;
+    }
+    // Unit i's streams (i >= nu: nothing to load).
+    WL_MEM void bind(uint32_t i, AS& A) {
+        const UnitInfo x = unit(i);
+        A.kd2 = 2u * (UP ? H : SI);
+        A.rs = make_rsrc(x.live ? (UP ? b.norm3 : b.smid3) : nullptr, x.live ? b.T * 3u * A.kd2 : 0u);
+        const uint32_t r0 = 4u * v + g, cg = n ^ (r0 & 15u);
+#pragma unroll
+        for (uint32_t j = 0; j < 2; j++) {
+            const uint32_t m = r0 + 32u * j;
+            A.base[j] = m < x.nt ? (x.row0 + m) * 3u * A.kd2 + 16u * cg : kOOBV;
+        }
+        const NativeShared NS = NativeShared::make(H, SI);
+        wpart = x.part;
+        wbase = !x.live ? nullptr : a.sh_native + (UP ? NS.sgu : NS.sdn);
+        wbytes = !x.live ? 0u : (uint32_t)(UP ? NS.sdn - NS.sgu : NS.total - NS.sdn);
+        if (!UP) {
+#pragma unroll
+            for (uint32_t t = 0; t < NT; t++)
+                vw[UP ? 0 : t] = (g * H + min(16u * (NT * (kGW * x.part + v) + t) + n, H - 1u)) * 16u;
+        }
+    }
+    template <int S>
+    WL_MEM void dma(const AS& A, uint32_t s, uint32_t j) const {
+        const uint32_t h = j % kRB2, pc = j / kRB2;
+        dma16<S>(A.rs, (16u * pc + 8u * h + v) * 1024u, A.base[h], 256u * s + pc * A.kd2);
+    }
+    WL_MEM void load(uint32_t s, WB& W, uint32_t j) const {
+        const rsrc_t rs = make_rsrc(wbase, wbytes);
+        const uint32_t t = j / 4u, k = j % 4u;
+        if (UP) W.w[j] = bld16(rs, vw[0], ((NT * (kGW * wpart + v) + t) * nkt + 4u * s + k) * 1024u);
+        else W.w[j] = bld16(rs, vw[UP ? 0 : t], (16u * s + 4u * k) * H * 16u);
+    }
+    WL_MEM void begin(uint32_t i) {
+        cu = unit(i);
+        const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (uint32_t t = 0; t < NT; t++)
+#pragma unroll
+            for (uint32_t m = 0; m < NB; m++) {
+                acc[t][m][0] = acc[t][m][1] = z;
+                if constexpr (kSum) sum[t][m] = z;
+            }
+    }
+    // Iteration it = 3 k + pc: plane pc of k step k (columns 32 k + 8 g of the
+    // step, group cg = 4 k + g: lane offset lob ^ 64 k) against the tiles; the
+    // next iteration's NB fragments are read while this one's MFMAs run.
+    template <class Next>
+    WL_MEM void comp(uint32_t, const uint8_t* sl, WB& W, Next next) {
+        auto frag = [&](uint32_t it, uint32_t m) {
+            return as_bf16x8(*(const u32x4*)(sl + ((it % 3u) * 64u + m * 16u) * 256u + (lob ^ (64u * (it / 3u)))));
+        };
+        bf16x8 af[2][NB];
+#pragma unroll
+        for (uint32_t m = 0; m < NB; m++) af[0][m] = frag(0u, m);
+#pragma unroll
+        for (uint32_t it = 0; it < 12u; it++) {
+            const uint32_t k = it / 3u, pc = it % 3u;
+            if (it + 1u < 12u) {
+#pragma unroll
+                for (uint32_t m = 0; m < NB; m++) af[(it + 1u) & 1u][m] = frag(it + 1u, m);
+            }
+            next(it, 12u);
+#pragma unroll
+            for (uint32_t t = 0; t < NT; t++) {
+                const bf16x8 bw = as_bf16x8(W.w[4u * t + k]);
+#pragma unroll
+                for (uint32_t m = 0; m < NB; m++) {
+                    const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+                    f32x4& c = acc[t][m][pc ? 1 : 0];
+                    c = mma(bw, af[it & 1u][m], kSum && it == 0u ? z : c);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (kSum) {
+#pragma unroll
+            for (uint32_t t = 0; t < NT; t++)
+#pragma unroll
+                for (uint32_t m = 0; m < NB; m++) sum[t][m] += acc[t][m][0];
+        }
+    }
+    WL_MEM f32x4 total(uint32_t t, uint32_t m) const {
+        if constexpr (kSum) return sum[t][m] + acc[t][m][1];
+        else return acc[t][m][0] + acc[t][m][1];
+    }
+    WL_MEM void finish() {
+        const uint32_t ln = opaque_lane(), nn = ln & 15u, gg = ln >> 4;
+        const uint32_t T0 = NT * (kGW * cu.part + v);
+        if constexpr (UP) {
+            // pairs of tiles, or of row blocks of the one tile
+            constexpr uint32_t NP = NT == 1u ? (NB + 1u) / 2u : NB;
+#pragma unroll
+            for (uint32_t m = 0; m < NP; m++) {
+                const uint32_t m0 = NT == 1u ? 2u * m : m, m1 = NT == 1u ? (2u * m + 1u < NB ? 2u * m + 1u : m0) : m;
+                const f32x4 x = swiglu_pair(total(0u, m0), total(NT - 1u, m1));
+                const float xs[4] = {x[0], x[1], x[2], x[3]};
+                const uint32_t r = 16u * (NT == 1u ? 2u * m + (gg >> 1) : m) + nn;
+                const uint32_t col = 8u * T0 + (NT == 1u ? 4u * (gg & 1u) : 4u * gg);
+                if (r < cu.nt) store_pieces4(b.smid3 + (size_t)(cu.row0 + r) * 3u * SI + col, SI, xs);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+#pragma unroll
+            for (uint32_t m = 0; m < NB; m++) {
+                const uint32_t r = 16u * m + nn;
+#pragma unroll
+                for (uint32_t t = 0; t < NT; t++) {
+                    const uint32_t row = 16u * (T0 + t) + 4u * gg;
+                    if (r < cu.nt && row < H) gst((f32x4*)(b.shout + (size_t)(cu.row0 + r) * H + row), total(t, m));
+                }
+            }
+        }
+    }
+};
+// Its units start at work-group 0; returns their count.
+template <bool UP, uint32_t NT, uint32_t NB>
+WL_DEV uint32_t run_shared(const DecodeArgs& a, const BatchArgs& b) {
+    SharedK<UP, NT, NB> k{a, b};
+    k.H = a.H;
+    k.SI = a.SI;
+    k.nkt = a.H / 32u;
+    k.parts = UP ? a.SI / (8u * kGW * NT) : cdiv(a.H, 16u * kGW * NT);
+    k.npass = cdiv(b.T, 64u);
+    k.nst = (UP ? a.H : a.SI) / 128u;
+    const uint32_t U = k.npass * k.parts, lane = threadIdx.x & 63u;
+    k.nu = U > blockIdx.x ? cdiv(U - blockIdx.x, gridDim.x) : 0u;
+    k.n = lane & 15u;
+    k.g = lane >> 4;
+    k.v = uni(threadIdx.x >> 6);
+    if (UP) k.vw[0] = 16u * lane;
+    k.lob = k.n * 256u + 16u * (k.g ^ k.n);
+    run_units(k);
+    return U;
+}
+// (More than two passes: the largest has at least 43 tokens, so three row
+// blocks or four.)
+template <bool UP>
+WL_DEV uint32_t run_shared_expert(const DecodeArgs& a, const BatchArgs& b) {
+    if (b.flags & (kBatchNoShared | kBatchShared4)) return 0u;
+    const uint32_t np = cdiv(b.T, 64u), nb = cdiv(cdiv(b.T, np), kRB);
+    if (np > 2u) return nb == 3u ? run_shared<UP, 2, 3>(a, b) : run_shared<UP, 2, 4>(a, b);
+    switch (nb) {
+        case 1: return run_shared<UP, 1, 1>(a, b);
+        case 2: return run_shared<UP, 1, 2>(a, b);
+        case 3: return run_shared<UP, 1, 3>(a, b);
+        default: return run_shared<UP, 1, 4>(a, b);
+    }
+}
+
+// ---- routed experts (MXFP4) ---------------------------------------------------------------
+// On rows quantised by q6.h.
+//
+// w: 16 weight rows of 128 columns in MXFP4, x: one piece of 16 tokens; byte ow
+// of sw and byte ox of sx are the lane's block scales (compile-time constants
+// after unrolling).
+WL_DEV f32x4 mmq(u32x4 w, i32x8 x, f32x4 c, uint32_t ow, uint32_t sw, uint32_t ox, uint32_t sx) {
+    const i32x8 A = {(int)w.x, (int)w.y, (int)w.z, (int)w.w, 0, 0, 0, 0};
+#define WL_MMQ(i, j) \
+    case 4 * i + j: return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, x, c, 4, 2, i, (int)sw, j, (int)sx)
+    switch (4u * ow + ox) {
+        WL_MMQ(0, 0); WL_MMQ(0, 1); WL_MMQ(0, 2); WL_MMQ(0, 3);
+        WL_MMQ(1, 0); WL_MMQ(1, 1); WL_MMQ(1, 2); WL_MMQ(1, 3);
+        WL_MMQ(2, 0); WL_MMQ(2, 1); WL_MMQ(2, 2); WL_MMQ(2, 3);
+        WL_MMQ(3, 0); WL_MMQ(3, 1); WL_MMQ(3, 2); WL_MMQ(3, 3);
+    }
+#undef WL_MMQ
+    return c;
+}
+// Piece p of a staged k tile of 16 rows at `tile`; lo8: the lane's offset of
+// its 8-byte parts.
+WL_DEV uint32_t q_lo8() {
+    const uint32_t lane = threadIdx.x & 63u, n = lane & 15u, g = lane >> 4;
+    return 256u * (g >> 1) + 16u * n + 8u * (g & 1u);
+}
+template <uint32_t P>
+WL_DEV i32x8 q_frag(const uint8_t* tile, uint32_t p, uint32_t lane16, uint32_t lo8) {
+    const u32x4 h = *(const u32x4*)(tile + 1024u * p + lane16);
+    const u32x2 l = *(const u32x2*)(tile + 1024u * P + 512u * p + lo8);
+    return i32x8{(int)h.x, (int)h.y, (int)h.z, (int)h.w, (int)l.x, (int)l.y, 0, 0};
+}
+template <uint32_t P>
+WL_DEV u32x2 q_scales(const uint8_t* tile, uint32_t lo8) {
+    return *(const u32x2*)(tile + 1536u * P + lo8);
+}
+// Two chunks of 64 columns of a row pair (lane (n, g): row 32 q + n + 16 (g >>
+// 1), block g & 1) -> 128 columns of each of its halves, in place.
+WL_DEV void pair_swap(u32x4& x, u32x4& y) {
+#pragma unroll
+    for (uint32_t d = 0; d < 4; d++) {
+        uint32_t lo, hi;
+        swap32(x[d], y[d], lo, hi);
+        x[d] = lo;
+        y[d] = hi;
+    }
+}
+
+// MB row blocks, KT k tiles per step: the slot holds tile (q, m), number MB q + m.
+// A DMA of a tile fills units c = 4u .. 4u + 3 of its 16 rows: lane (n, g) reads
+// 16 bytes of row 16 m + n, at its base + 64 u. Wave v takes u = v of every tile;
+// of a record of ten such groups, the two left over of four tiles at once: wave
+// v group 8 + v % 2 of tile 4 x + v / 2 (past the tiles: out of range, into the
+// slot's end). Absent rows, k tiles past the row's end and units past the record
+// land as zeros (zero scales too: their products are zero).
+template <uint32_t MB>
+struct AStreamQ {
+    rsrc_t rs;
+    uint32_t base[MB], left, nk;  // lane byte offsets of the lane's rows (left: of its left-over groups' row), k tiles of a row
+};
+// What the pipelines share: the layer's tables, the rows of a pass, the
+// epilogues. UP: gate/up of the routed experts, K = H, slices of 64 rows (tiles of
+// 8 gate and 8 up rows), SwiGLU values to midf.
+// Otherwise down, K = I, row pairs (rows 32 q + n and + 16), to expout. A unit
+// is four slices, or 16 row pairs: four tiles per wave (tile 8 sl + v of slice
+// sl, row pairs 2 v and 2 v + 1 of the 16), as the native block's batched scale
+// words are laid out. NB row blocks, KT k tiles per step.
+template <bool UP, uint32_t NB, uint32_t KT>
+struct QBase {
+    using AS = AStreamQ<NB>;
+    static constexpr uint32_t P = UP ? kQPUp : kQPDown, NG = (q6_units(P) + 3u) / 4u;  // groups of a record
+    static constexpr uint32_t kTiles = NB * KT, kTileB = 1024u * NG, kLeft = NG > 8u ? (kTiles + 3u) / 4u : 0u;
+    static constexpr uint32_t kDmas = kTiles + kLeft;
+    static_assert(NG == 8u || (NG == 10u && kLeft == 1u), "eight groups, or ten of at most four tiles");
+    static_assert(kTileB * kTiles + (kLeft ? 8192u : 0u) <= kSlotB, "a step's tiles fit a slot");
+    const DecodeArgs& a;
+    const BatchArgs& b;
+    uint32_t H, I, E, K, nk, S, nq, parts, nst, nst2, nu, v, lane, g, uoff;
+    PassTab pt;
+    const uint8_t* const* stab;
+    NativeLayout NL;
+    Cursor cn, cc;  // positions of the loads and of the compute
+    const uint8_t* wbase;  // the weight stream's block and size (see SharedK)
+    uint32_t wbytes, wpart, vw, vs, lo8;
+    UnitInfo cu, un;     // the unit computed, the unit whose loads go out
+    const uint16_t *tt, *ent;  // UP: the token table; the entries where this kernel grouped them (or null)
+
+    WL_MEM UnitInfo unit(uint32_t i) const {
+        UnitInfo x{false, 0u, 0u, 0u, 0u};
+        if (i >= nu) return x;
+        const uint32_t u = (blockIdx.x + gridDim.x - uoff) % gridDim.x + gridDim.x * i;
+        const PassPart jp = pass_part(u, parts, pt.n);
+        const Pass ps = pass_at(pt, E, jp.j);
+        x.live = true;
+        x.part = jp.part;
+        x.e = ps.e;
+        x.nt = ps.nt;
+        x.row0 = ps.c0;
+        return x;
+    }
+    WL_MEM void bind(uint32_t i, AS& A) {
+        const UnitInfo x = un = unit(i);
+        const uint8_t* blk = x.live ? uni_ptr(stab[x.e]) : nullptr;
+        wbase = blk;
+        wbytes = blk ? (uint32_t)NL.total : 0u;
+        wpart = x.part;
+        const uint32_t kd = UP ? H : I, n = lane & 15u;
+        const uint32_t nrow = UP ? b.T : b.T * (K + ((b.flags & kBatchShared4) ? 1u : 0u));
+        const uint32_t rowb = (uint32_t)q6_row_bytes(P, kd);
+        A.rs = make_rsrc(x.live ? (UP ? (const uint8_t*)b.norm : b.mid6) : nullptr, x.live ? nrow * rowb : 0u);
+        A.nk = x.live ? nk : 0u;
+        auto row_at = [&](uint32_t m) {
+            const uint32_t r = kRB * m + n;
+            uint32_t row = x.row0 + r;
+            if (UP) row = x.e == a.E ? row - b.T * K : x.live ? table_token(tt, b.tcap, kRB * NB, i, r, x.nt) : 0u;
+            return r < x.nt ? row * rowb + 16u * g : kOOBV;
+        };
+#pragma unroll
+        for (uint32_t m = 0; m < NB; m++) {
+            const uint32_t o = row_at(m);
+            A.base[m] = o == kOOBV ? o : o + 64u * v;
+        }
+        if (kLeft) {
+            const uint32_t c = 4u * (8u + v % 2u) + g, o = row_at(v / 2u % NB);
+            A.left = v / 2u < kTiles && c < q6_units(P) && o != kOOBV ? o + 64u * (8u + v % 2u) : kOOBV;
+        }
+    }
+    template <int SL>
+    WL_MEM void dma(const AS& A, uint32_t s, uint32_t j) const {
+        if (j < kTiles) {
+            const uint32_t k = s * KT + j / NB;
+            dma16<SL>(A.rs, j * kTileB + v * 1024u, k < A.nk ? A.base[j % NB] : kOOBV, k * q6_record(P));
+        } else {
+            const uint32_t t = v / 2u, k = s * KT + t / NB;
+            dma16<SL>(A.rs, t < kTiles ? t * kTileB + (8u + v % 2u) * 1024u : kTiles * kTileB + v * 1024u,
+                      k < A.nk ? A.left : kOOBV, k * q6_record(P));
+        }
+    }
+    WL_MEM void begin_unit(uint32_t i) {
+        cu = nst > 1u && i > 0u ? un : unit(i);  // (the loads are two steps ahead)
+        if (cu.live && stab[cu.e] == nullptr && threadIdx.x == 0) raise_error(a.sync, SyncMap::make(), E_NOT_RESIDENT, 0u);  // no waits in this path: epoch 0 aborts nothing
+    }
+    // The four slices of row block m, two at a time.
+    template <class D>
+    WL_MEM void put_up(uint32_t m, D d) const {
+        const uint32_t ln = opaque_lane(), r = kRB * m + (ln & 15u), gg = ln >> 4;
+        float* o = b.midf + (size_t)(cu.row0 + r) * b.ldm + 8u * v + 4u * (gg & 1u);
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i += 2) {
+            const uint32_t sl = cu.part * 4u + i + (gg >> 1);
+            const f32x4 x = swiglu_pair(d(i), d(i + 1u));
+            if (r < cu.nt && sl < S) gst((f32x4*)(o + sl * kSlice), x);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    WL_MEM void put_down(const f32x4& d, uint32_t m, uint32_t q, uint32_t h) const {
+        const uint32_t ln = opaque_lane(), r = kRB * m + (ln & 15u);
+        if (r < cu.nt && q < nq) gst((f32x4*)(b.expout + (size_t)(cu.row0 + r) * b.ldm + 32u * q + 16u * h + 4u * (ln >> 4)), d);
+    }
+};
+
+// Passes of one or two row blocks: bound by the weight stream (a step is 64 KB
+// of weights against at most 3600 cycles of MFMA per SIMD); a step has 256
+// columns: per wave 8 chunks of 1 KB and the batched scale word (bgus, bdns). UP:
+// 4 slices x 2 k tiles; down: 4 slices of 64 columns x 2 row pairs. The first piece and the
+// others sum in accumulators of their own; in passes of one row block the first
+// piece's are added to the sums at every step in f32 (matrix instructions that
+// add into a large sum round it more coarsely).
+template <bool UP, uint32_t NB>
+struct QNarrow : QBase<UP, NB, 2> {
+    using QB = QBase<UP, NB, 2>;
+    using QB::P;
+    struct WB {
+        u32x4 w[8];
+        uint32_t s[2];
+    };
+    static constexpr uint32_t kLoads = 9;
+    static constexpr bool kSum = NB == 1u;
+    f32x4 acc[4][NB][2], sum[kSum ? 4 : 1];
+
+    WL_MEM QNarrow(const DecodeArgs& a_, const BatchArgs& b_) : QB{a_, b_} {}
+    WL_MEM void load(uint32_t s, WB& W, uint32_t j) const {
+        const rsrc_t rs = make_rsrc(this->wbase, this->wbytes);
+        if (j == 8u) return bld8(rs, this->vs, (this->wpart * 8u * this->nst2 + s) * 512u, W.s);
+        uint32_t ch;
+        if (UP) ch = min(this->wpart * 4u + j / 2u, this->S - 1u) * 8u * this->nk + min(2u * s + j % 2u, this->nk - 1u);
+        else ch = min(4u * s + j / 2u, 2u * this->nk - 1u) * this->nq + min(16u * this->wpart + 2u * this->v + j % 2u, this->nq - 1u);
+        W.w[j] = bld16_nt(rs, this->vw, ch * 1024u);
+    }
+    WL_MEM void begin(uint32_t i) {
+        this->begin_unit(i);
+        const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (uint32_t t = 0; t < 4; t++) {
+#pragma unroll
+            for (uint32_t m = 0; m < NB; m++) acc[t][m][0] = acc[t][m][1] = z;
+            if (kSum) sum[t] = z;
+        }
+    }
+    // Operands it = (P q + p) NB + m in this order; each runs against the wave's
+    // weight tiles while the two after it are read.
+    template <class Next>
+    WL_MEM void comp(uint32_t, const uint8_t* sl, WB& W, Next next) {
+        constexpr uint32_t N = 2u * P * NB, AH = 2u;
+        i32x8 af[AH + 1u];
+        u32x2 sa[NB];
+        uint32_t sx = 0u, sy = 0u;
+        const uint32_t lane16 = 16u * this->lane;
+        auto tile = [&](uint32_t q, uint32_t m) { return sl + (q * NB + m) * QB::kTileB; };
+        auto frag = [&](uint32_t it) {
+            const uint32_t m = it % NB, p = it / NB % P, q = it / (NB * P);
+            return q_frag<P>(tile(q, m), p, lane16, this->lo8);
+        };
+#pragma unroll
+        for (uint32_t it = 0; it < AH; it++) af[it] = frag(it);
+#pragma unroll
+        for (uint32_t it = 0; it < N; it++) {
+            const uint32_t m = it % NB, p = it / NB % P, q = it / (NB * P);
+            if (p == 0u && m == 0u) {
+#pragma unroll
+                for (uint32_t i = 0; i < NB; i++) sa[i] = q_scales<P>(tile(q, i), this->lo8);
+                if (!UP) {
+#pragma unroll
+                    for (uint32_t h = 0; h < 2; h++) pair_swap(W.w[4u * q + h], W.w[4u * q + 2u + h]);
+                    swap32(W.s[q], W.s[q] >> 16, sx, sy);
+                }
+            }
+            if (it + AH < N) af[(it + AH) % (AH + 1u)] = frag(it + AH);
+            next(it, N);
+#pragma unroll
+            for (uint32_t t = 0; t < 4; t++) {
+                // UP: slice t; down: row pair t % 2, half t / 2
+                const uint32_t ow = UP ? 2u * (t & 1u) + q : t & 1u;
+                const uint32_t sw = UP ? W.s[t >> 1] : (t & 2u) ? sy : sx;
+                const u32x4 w = W.w[UP ? 2u * t + q : 4u * q + t];
+                const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+                f32x4& c = acc[t][m][p == 0u ? 0u : 1u];
+                c = mmq(w, af[it % (AH + 1u)], kSum && p == 0u && q == 0u ? z : c, ow, sw, p & 3u, p < 4u ? sa[m].x : sa[m].y);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (kSum) {
+#pragma unroll
+            for (uint32_t t = 0; t < 4; t++) sum[t] += acc[t][0][0];
+        }
+    }
+    WL_MEM void finish() {
+#pragma unroll
+        for (uint32_t m = 0; m < NB; m++) {
+            auto d = [&](uint32_t t) {
+                if constexpr (kSum) return sum[t] + acc[t][0][1];
+                else return acc[t][m][0] + acc[t][m][1];
+            };
+            if constexpr (UP) {
+                this->put_up(m, d);
+            } else {
+#pragma unroll
+                for (uint32_t t = 0; t < 4; t++) this->put_down(d(t), m, this->cu.part * 16u + 2u * this->v + (t & 1u), t >> 1);
+            }
+        }
+    }
+};
+
+// Passes of three to five row blocks (down: four, six pieces take more LDS): bound
+// by the matrix cores and the loads' issue (750 to 900 cycles of MFMA per SIMD and
+// row block for a step's 32 KB of weights and 8 to 10 KB of rows per block). A
+// step is 128 columns.
+template <bool UP, uint32_t NB>
+struct QWide : QBase<UP, NB, 1> {
+    using QB = QBase<UP, NB, 1>;
+    using QB::P;
+    struct WB {
+        u32x4 w[4];
+        uint32_t s[2];
+    };
+    static constexpr uint32_t kLoads = 5;
+    f32x4 acc[4][NB];
+
+    WL_MEM QWide(const DecodeArgs& a_, const BatchArgs& b_) : QB{a_, b_} {}
+    WL_MEM void load(uint32_t s, WB& W, uint32_t j) const {
+        const rsrc_t rs = make_rsrc(this->wbase, this->wbytes);
+        if (j < 4u) {
+            uint32_t ch;  // UP: slice j; down: slice 2s + (j & 1) of row pair j / 2
+            if (UP) ch = min(this->wpart * 4u + j, this->S - 1u) * 8u * this->nk + s;
+            else ch = (2u * s + j % 2u) * this->nq + min(16u * this->wpart + 2u * this->v + j / 2u, this->nq - 1u);
+            W.w[j] = bld16(rs, this->vw, ch * 1024u);
+        } else {
+            const uint32_t so = (this->wpart * 8u * this->nst2 + s / 2u) * 512u;
+            if (UP) bld8(rs, this->vs, so, W.s);
+            else W.s[0] = __builtin_amdgcn_raw_buffer_load_b32(rs, (int)this->vs, (int)(so + 4u * (s & 1u)), 0);
+        }
+    }
+    WL_MEM void begin(uint32_t i) {
+        this->begin_unit(i);
+#pragma unroll
+        for (uint32_t t = 0; t < 4; t++)
+#pragma unroll
+            for (uint32_t m = 0; m < NB; m++) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    template <class Next>
+    WL_MEM void comp(uint32_t s, const uint8_t* sl, WB& W, Next next) {
+        constexpr uint32_t N = P * NB, AH = 2u;
+        i32x8 af[AH + 1u];
+        u32x2 sa[NB];
+        const uint32_t lane16 = 16u * this->lane;
+        auto frag = [&](uint32_t it) { return q_frag<P>(sl + (it % NB) * QB::kTileB, it / NB, lane16, this->lo8); };
+#pragma unroll
+        for (uint32_t it = 0; it < AH; it++) af[it] = frag(it);
+#pragma unroll
+        for (uint32_t m = 0; m < NB; m++) sa[m] = q_scales<P>(sl + m * QB::kTileB, this->lo8);
+        // the step's scale bytes: UP the step's k tile of the word's two (byte 2
+        // (i & 1)), down as the weights' halves (byte h)
+        if (UP) {
+            W.s[0] >>= 8u * (s & 1u);
+            W.s[1] >>= 8u * (s & 1u);
+        } else {
+            uint32_t lo, hi;
+            swap32(W.s[0], W.s[0] >> 16, lo, hi);
+            W.s[0] = lo;
+            W.s[1] = hi;
+            pair_swap(W.w[0], W.w[1]);
+            pair_swap(W.w[2], W.w[3]);
+        }
+#pragma unroll
+        for (uint32_t it = 0; it < N; it++) {
+            const uint32_t m = it % NB, p = it / NB;
+            if (it + AH < N) af[(it + AH) % (AH + 1u)] = frag(it + AH);
+            next(it, N);
+#pragma unroll
+            for (uint32_t t = 0; t < 4; t++) {
+                // UP: slice t; down: row pair t / 2, half t % 2
+                const uint32_t ow = UP ? 2u * (t & 1u) : t >> 1;
+                const uint32_t sw = UP ? W.s[t >> 1] : W.s[t & 1u];
+                acc[t][m] = mmq(W.w[t], af[it % (AH + 1u)], acc[t][m], ow, sw, p & 3u, p < 4u ? sa[m].x : sa[m].y);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    WL_MEM void finish() {
+#pragma unroll
+        for (uint32_t m = 0; m < NB; m++) {
+            if constexpr (UP) {
+                this->put_up(m, [&](uint32_t t) { return acc[t][m]; });
+            } else {
+#pragma unroll
+                for (uint32_t t = 0; t < 4; t++) this->put_down(acc[t][m], m, 16u * this->cu.part + 2u * this->v + (t >> 1), t & 1u);
+            }
+        }
+    }
+};
+
+// Calls of at most kGroupMax entries that run all phases (BatchArgs::group): the
+// work-groups of bup_kernel find the experts' counts, offsets and entries from the
+// ids by themselves, one entry per thread (its rank: the entries of its expert
+// before it), and the first also stores them for the kernels after it. bcount and
+// bscatter, a launch of 5 us each, take all other calls.
+constexpr uint32_t kGroupMax = kGT;
+// The LDS of the grouped entries, after the token table.
+__host__ __device__ inline size_t ent_table_offset(uint32_t E, uint32_t tcap) { return tok_table_offset(E) + 2u * (size_t)tcap; }
+WL_DEV void group_entries(const BatchArgs& b, uint32_t E, uint32_t K, const ExpertTab& et, uint16_t* ent) {
+    const uint32_t n = b.T * K, i = threadIdx.x, lane = i & 63u;
+    uint32_t* ids = (uint32_t*)slot<0>();  // (free until the first pipeline)
+    const uint32_t id = i < n ? (uint32_t)gld(b.idx + i) : ~0u;
+    ids[i] = id;
+    for (uint32_t f = i; f < E; f += kGT) et.cnt[f] = 0u;
+    lds_barrier();
+    if (i < n) atomicAdd(et.cnt + id, 1u);
+    uint32_t rank = 0;
+    const uint32_t nb = min(n, uni(i | 63u) + 1u);  // (entries past n are no expert's)
+#pragma unroll 1
+    for (uint32_t j = 0; j < nb; j += 32u) {
+        u32x4 q[8];
+#pragma unroll
+        for (uint32_t r = 0; r < 8; r++) q[r] = *(const u32x4*)(ids + j + 4u * r);
+#pragma unroll
+        for (uint32_t r = 0; r < 32; r++) rank += q[r / 4u][r % 4u] == id && j + r < i ? 1u : 0u;
+    }
+    lds_barrier();
+    if (i < 64u) {
+        const uint32_t per = cdiv(E, 64u), e0 = lane * per;
+        uint32_t mine = 0;
+        for (uint32_t f = e0; f < min(e0 + per, E); f++) mine += et.cnt[f];
+        uint32_t inc = mine;
+#pragma unroll
+        for (uint32_t o = 1; o < 64u; o <<= 1) {
+            const uint32_t t = __shfl_up(inc, o, 64);
+            if (lane >= o) inc += t;
+        }
+        uint32_t off = inc - mine;
+        for (uint32_t f = e0; f < min(e0 + per, E); f++) {
+            et.off[f] = off;
+            off += et.cnt[f];
+        }
+    }
+    lds_barrier();
+    const bool put = blockIdx.x == 0u;
+    if (i < n) {
+        const uint32_t r = et.off[id] + rank;
+        ent[r] = (uint16_t)i;
+        if (put) {
+            gst(b.ent + r, i);
+            gst(b.pos + i, r);
+        }
+    }
+    if (!put) return;
+    for (uint32_t f = i; f < E; f += kGT) {
+        gst(b.counts + f, et.cnt[f]);
+        gst(b.offsets + f, et.off[f]);
+    }
+    if (i == 0u) gst(b.offsets + E, n);
+}
+WL_DEV ExpertTab load_expert_tab(const BatchArgs& b, uint32_t E, uint32_t K, uint32_t* s, const uint8_t* const* stab,
+                                 bool up) {
+    const ExpertTab et{s, s + E, s + 2u * E};
+    const bool skip = (b.flags & kBatchSkipUnbound) != 0u;
+    const uint32_t esh = (b.flags & kBatchShared4) ? E - 1u : E;
+    const bool group = up && b.group != 0u;
+    if (group) group_entries(b, esh, K, et, (uint16_t*)(dyn_lds() + ent_table_offset(esh, b.tcap)));
+    for (uint32_t f = threadIdx.x; f < E; f += kGT) {
+        if (f == esh) {
+            et.cnt[f] = (b.flags & kBatchNoShared) ? 0u : b.T;
+            et.off[f] = b.T * K;
+            continue;
+        }
+        if (group) continue;
+        // stab[f] was written by this thread (load_slot_tab, same stride)
+        et.cnt[f] = skip && stab[f] == nullptr ? 0u : gld(b.counts + f);
+        et.off[f] = gld(b.offsets + f);
+    }
+    return et;
+}
+// The routed passes of NB row blocks, starting at work-group uoff; returns
+// their units' count.
+template <bool UP, uint32_t NB>
+WL_DEV uint32_t run_routed(const DecodeArgs& a, const BatchArgs& b, uint32_t E, const ExpertTab& et,
+                           const uint8_t* const* stab, uint32_t uoff) {
+    using Kn = std::conditional_t<(NB > 2u), QWide<UP, NB>, QNarrow<UP, NB>>;
+    const PassTab pt = load_pass_tab(et, E, UP ? kWideUp : kWideDown, NB);
+    if (pt.n == 0u) return 0u;
+    pipeline_drain();
+    const uint32_t H = a.H, I = a.I;
+    Kn w(a, b);
+    w.H = H;
+    w.I = I;
+    w.E = E;
+    w.K = a.K;
+    w.nk = (UP ? H : I) / 128u;
+    w.S = I / kSlice;
+    w.nq = H / 32u;
+    w.parts = UP ? cdiv(w.S, 4u) : cdiv(w.nq, 16u);
+    w.nst2 = cdiv(UP ? H : I, 256u);
+    w.nst = NB > 2u ? w.nk : w.nst2;
+    w.uoff = uoff % gridDim.x;
+    const uint32_t U = pt.n * w.parts, b0 = (blockIdx.x + gridDim.x - w.uoff) % gridDim.x;
+    w.nu = U > b0 ? cdiv(U - b0, gridDim.x) : 0u;
+    w.lane = threadIdx.x & 63u;
+    w.g = w.lane >> 4;
+    w.v = uni(threadIdx.x >> 6);
+    w.lo8 = q_lo8();
+    w.pt = pt;
+    w.stab = stab;
+    w.NL = NativeLayout::make(H, I);
+    w.vw = (UP ? (uint32_t)w.NL.gu + w.v * w.nk * 1024u : (uint32_t)w.NL.dn) + 16u * w.lane;
+    w.vs = (uint32_t)(UP ? w.NL.bgus : w.NL.bdns) + w.v * w.nst2 * 512u + 8u * w.lane;
+    if (UP) {
+        uint16_t* tt = (uint16_t*)(dyn_lds() + tok_table_offset(a.E));
+        w.tt = tt;
+        w.ent = b.group ? (const uint16_t*)(dyn_lds() + ent_table_offset(a.E, b.tcap)) : nullptr;
+        fill_tokens(w, tt, kRB * NB);
+    }
+    run_units(w);
+    return U;
+}
+// The layer's units: the shared expert's, then the routed passes from the largest.
+// Routed rows as fp6 pieces against fp4 weights run at 3.5 times the rate of bf16
+// pieces and need no conversion of the weights. Whole calls, hidden 6144, inter
+// 2048, 8 of 256 experts (256 work-groups of eight waves), before (bf16 pieces,
+// passes of 32 and 64) and now: 4096 tokens 8440 and 4940 us, 1000 tokens 2310 and
+// 1585, 64 tokens (one row block per expert; the weights' 4.4 GB at 6 TB/s) 724 and
+// 739, 7 tokens 213.0 and 214.4; hidden 2944, inter 1408, 6 of 160 experts, 333 tokens: 457 and 310.
+// Error against 64 bits: 8.1e-7 and 4.5e-7 at 4096 tokens, 3.5e-7 and 1.5e-7 at 64.
+template <bool UP>
+WL_DEV void run_gemm(const DecodeArgs* pa, const BatchArgs& b) {
+    const DecodeArgs& a = *pa;
+    uint8_t* dyn = dyn_lds();
+    const bool sh4 = (b.flags & kBatchShared4) != 0u;
+    const uint32_t E = a.E + (sh4 ? 1u : 0u);  // experts in the pass table
+    const uint8_t* const* stab = load_slot_tab(a, a.E, sh4, (const uint8_t**)dyn);
+    const ExpertTab et = load_expert_tab(b, E, a.K, (uint32_t*)(dyn + 8u * E), stab, UP);
+    uint32_t u = run_shared_expert<UP>(a, b);
+    if constexpr (UP) u += run_routed<UP, 5>(a, b, E, et, stab, u);
+    u += run_routed<UP, 4>(a, b, E, et, stab, u);
+    u += run_routed<UP, 3>(a, b, E, et, stab, u);
+    u += run_routed<UP, 2>(a, b, E, et, stab, u);
+    run_routed<UP, 1>(a, b, E, et, stab, u);
+}

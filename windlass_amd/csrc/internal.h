@@ -277,24 +277,13 @@ struct NativeShared4 {
 // (a source-backed layer runs its routed set in chunks of experts); the
 // shared expert's units are left out (they run with the first chunk only).
 // kBatchShared4: the shared expert is MXFP4 and runs as expert E of the pass
-// table (all T tokens, activations straight from norm3, outputs in the rows
-// [T*K, T*K + T) of mid3 and expout).
-// kBatchWideSharedUp / Down (set by launch_batched): the bf16 shared
-// expert's gate/up (down) runs as 64-token units in the wide GEMM kernel.
+// table (all T tokens, activations straight from norm, outputs in the rows
+// [T*K, T*K + T) of midf, mid6 and expout).
 enum : uint32_t {
     kBatchSkipUnbound = 1u,
     kBatchNoShared = 2u,
-    kBatchShared4 = 4u,
-    kBatchWideSharedUp = 8u,
-    kBatchWideSharedDown = 16u
+    kBatchShared4 = 4u
 };
-// Routed experts of few tokens run their gate/up and down projections in the
-// GEMM kernels' streaming pipelines (run_small_up, run_small_down) when
-// launch_batched takes those kernels' small-expert instantiations (at the
-// shapes they fit): 1..kSmallT tokens in one MFMA row block, and at the GLM
-// shape kSmallT+1..kSmallUpT (moe_batched.hip) in two; their pass tables leave
-// them out of the other pipelines.
-constexpr uint32_t kSmallT = 4;
 // launch_batched phases: routing (norm .. scatter), the GEMMs, the combine.
 enum : uint32_t { kPhaseRoute = 1u, kPhaseGemm = 2u, kPhaseCombine = 4u, kPhaseAll = 7u };
 struct BatchArgs {
@@ -303,7 +292,7 @@ struct BatchArgs {
     const float* hidden;   // [T][H] pre-norm residual stream
     const float* resid;    // [T][H] or null
     float* out;            // [T][H]
-    float* norm;           // [T][H]
+    float* norm;           // [T][H]; after the top-k its quantised rows (q6.h: as many bytes)
     uint16_t* norm3;       // [T][3][H] bf16 pieces of norm
     float* logits;         // [T][E]
     int32_t* idx;          // [T][K]
@@ -313,15 +302,15 @@ struct BatchArgs {
     uint32_t* lists;       // [E][T] entries (token*K + slot) of expert e, ascending
     uint32_t* ent;         // [T*K] compact index -> token*K + slot (expert-major)
     uint32_t* pos;         // [T*K] token*K + slot -> compact index
-    uint16_t* mid3;        // [T*K (+T)][3][I] routed (and MXFP4 shared) SwiGLU outputs (pieces), compact rows
+    uint8_t* mid6;         // [T*K (+T)] quantised rows of midf (q6.h)
+    uint32_t ldm;          // stride of the rows of midf and expout, which share their space row by row
+    float* midf;           // [T*K (+T)][I] routed (and MXFP4 shared) SwiGLU outputs, compact rows
     float* expout;         // [T*K (+T)][H] routed (and MXFP4 shared) expert outputs, compact rows
     uint16_t* smid3;       // [T][3][SI] shared SwiGLU outputs (pieces)
     float* shout;          // [T][H]
     uint32_t tcap;         // token-table entries per work-group in bup_kernel's LDS (set by launch_batched)
-    uint32_t* wq;          // [kWqWords] work-queue counters of the streaming units: zero between launches
-                           // (zeroed once when the scratch is made, reset by each launch's last work-group)
+    uint32_t group;        // bup_kernel groups the entries by expert itself (set by launch_batched)
 };
-constexpr uint32_t kWqWords = 8;
 
 // Launchers (moe_decode.hip).
 int launch_decode(const DecodeArgs* d_args, const DecodeDyn& dyn, uint32_t H, uint32_t I, uint32_t SI,
@@ -373,7 +362,7 @@ uint32_t batched_max_experts();
 // Largest batched chunk (tokens per launch) whose gate/up token table fits in
 // LDS beside the activation slots and the expert tables, for a grid of at
 // least `grid` work-groups.
-uint32_t batched_max_tokens(uint32_t I, uint32_t SI, uint32_t E, uint32_t K, uint32_t grid);
+uint32_t batched_max_tokens(uint32_t I, uint32_t E, uint32_t K, uint32_t grid);
 int launch_batched(const DecodeArgs* d_args, const BatchArgs& b, uint32_t H, uint32_t I, uint32_t SI, uint32_t E,
                    uint32_t K, uint32_t n_cu, uint32_t phases, void* stream);
 // The library's static device scratch (noalloc.hip): its device address on

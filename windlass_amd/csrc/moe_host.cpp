@@ -1105,7 +1105,6 @@ static size_t batch_layout(const wl_ctx* c, uint32_t T, uint8_t* base, wl::Batch
     };
     wl::BatchArgs d{};
     wl::BatchArgs& x = b ? *b : d;
-    take(&x.wq, 4 * wl::kWqWords);  // first: the same offset in every layout of the shared static scratch
     take(&x.norm, 4 * t * H);
     take(&x.norm3, 6 * t * H);
     take(&x.logits, 4 * t * E);
@@ -1117,8 +1116,12 @@ static size_t batch_layout(const wl_ctx* c, uint32_t T, uint8_t* base, wl::Batch
     take(&x.ent, 4 * t * K);
     take(&x.pos, 4 * t * K);
     const size_t Kr = K + (c->any_sh4 ? 1u : 0u);  // + the MXFP4 shared expert's rows
-    take(&x.mid3, 6 * t * Kr * I);
-    take(&x.expout, 4 * t * Kr * H);
+    take(&x.mid6, 6 * t * Kr * I);  // (records of 4.75 bytes per value; this size keeps the chunks of the static scratch)
+    // a row's SwiGLU values are read before its output is written (and no
+    // other row's output lies there): they share its space
+    x.ldm = (uint32_t)std::max(I, H);
+    take(&x.expout, 4 * t * Kr * x.ldm);
+    x.midf = x.expout;
     take(&x.smid3, 6 * t * SI);
     take(&x.shout, 4 * t * H);
     return (o + 255u) & ~(size_t)255u;
@@ -1149,8 +1152,6 @@ static wl_status batch_reserve(wl_ctx* c, uint32_t T) {
         return fail(c, WL_ERR_OOM, "batched scratch for %u tokens (%zu B)", T, bytes);
     }
     batch_layout(c, T, (uint8_t*)B.buf, &B.b);
-    if ((e = hipMemset(B.b.wq, 0, 4 * wl::kWqWords)) != hipSuccess || (e = hipDeviceSynchronize()) != hipSuccess)
-        return hip_fail(c, e, "batched work-queue words");
     B.cap = T;
     B.sh4 = c->any_sh4;
     return WL_OK;
@@ -1193,8 +1194,8 @@ static wl_status batched_check(wl_ctx* c, uint32_t layer, uint32_t n_tokens, con
 static uint32_t batch_offset_cap(const wl_ctx* c) {
     const uint64_t H = c->cfg.hidden, K = c->cfg.n_experts_per_tok + (c->any_sh4 ? 1u : 0u);
     const uint64_t row = 6ull * K * std::max<uint64_t>(std::max<uint64_t>(H, c->cfg.moe_inter), c->SI);
-    const uint32_t lds = wl::batched_max_tokens(c->cfg.moe_inter, c->SI, c->cfg.n_routed_experts,
-                                                c->cfg.n_experts_per_tok, (uint32_t)c->n_cu);
+    const uint32_t lds = wl::batched_max_tokens(c->cfg.moe_inter, c->cfg.n_routed_experts, c->cfg.n_experts_per_tok,
+                                                (uint32_t)c->n_cu);
     return (uint32_t)std::min<uint64_t>(std::min<uint64_t>(kBatchChunk, lds), ((1ull << 31) - 1) / row);
 }
 
