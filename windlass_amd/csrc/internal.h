@@ -365,6 +365,19 @@ uint32_t batched_max_experts();
 uint32_t batched_max_tokens(uint32_t I, uint32_t E, uint32_t K, uint32_t grid);
 int launch_batched(const DecodeArgs* d_args, const BatchArgs& b, uint32_t H, uint32_t I, uint32_t SI, uint32_t E,
                    uint32_t K, uint32_t n_cu, uint32_t phases, void* stream);
+// The dense MLP over T positions (batched_dense.h). scratch: T *
+// dense_token_bytes(H, DI) bytes, 16-byte aligned.
+constexpr uint32_t kDenseS = 8;  // K splits of down at most
+struct DenseBatch {
+    const float *hidden, *resid;
+    float* out;
+    const uint16_t *ln, *gate, *up, *down;
+    uint32_t T, H, DI;
+    float eps;
+    float* tap;  // the last position's normalised row, or null
+};
+uint64_t dense_token_bytes(uint32_t H, uint32_t DI);
+int launch_dense_batched(const DenseBatch& x, uint32_t n_cu, void* scratch, void* stream);
 // The library's static device scratch (noalloc.hip): its device address on
 // `device` (which must be current), looked up once per device and kept;
 // and its size in bytes.

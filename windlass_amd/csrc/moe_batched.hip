@@ -486,6 +486,7 @@ WL_DEV void bld8(rsrc_t r, uint32_t voff, uint32_t soff, uint32_t (&s)[2]) {
 }
 
 #include "batched_gemm.h"
+#include "batched_dense.h"
 
 // The gate/up and down projections of every expert (persistent: the grid is
 // what the chip holds at once, one work-group per CU).
@@ -643,6 +644,57 @@ int launch_batched(const DecodeArgs* d_args, const BatchArgs& b, uint32_t H, uin
     }
     if (phases & kPhaseCombine)
         hipLaunchKernelGGL(bcomb_kernel, dim3((H + 1023) / 1024, b.T), dim3(256), 0, s, b, H, K);
+    return (int)hipGetLastError();
+}
+
+uint64_t dense_token_bytes(uint32_t H, uint32_t DI) { return 6ull * H + 6ull * DI + 4ull * kDenseS * H; }
+int launch_dense_batched(const DenseBatch& x, uint32_t n_cu, void* scratch, void* stream) {
+    hipStream_t s = (hipStream_t)stream;
+    auto cd = [](uint64_t a, uint64_t b) { return (a + b - 1u) / b; };
+    // Passes and splits, in steps of a work-group (128 columns; 1.3 us with four
+    // row blocks): its rounds of units times a unit's steps and about two for its
+    // start, down also the partial rows written and read back at 5 TB/s. (200
+    // positions of hidden 6144, inter 12288: five passes of 40 make 480 gate/up
+    // units of three row blocks, two rounds of 256; four of 50 two rounds of four
+    // row blocks.)
+    uint32_t np = 0, S = 1;
+    double best = 0.0;
+    const uint64_t kup = cd(x.H, 128u), kdn = cd(x.DI, 128u);
+    for (uint64_t p = cd(x.T, 64u); p <= cd(x.T, 16u); p++) {
+        const double c = (double)(cd(cd(x.DI, 128u) * p, n_cu) * (kup + 2u)) * (1.0 + (double)cd(cd(x.T, p), kRB));
+        if (np == 0u || c < best) {
+            best = c;
+            np = (uint32_t)p;
+        }
+    }
+    for (uint32_t k = 1; k <= kDenseS; k++) {
+        const double c = (double)(cd(cd(x.H, 256u) * np * k, n_cu) * (cd(kdn, k) + 2u)) + (double)k * x.T * x.H / 8.5e5;
+        if (k == 1u || c < best) {
+            best = c;
+            S = k;
+        }
+    }
+    DenseArgs d{x.hidden, x.resid, x.out, x.ln, x.gate, x.up, x.down, x.T, x.H, x.DI, np, S, x.eps, x.tap,
+                (uint16_t*)scratch, nullptr, nullptr};
+    d.mid3 = d.norm3 + 3ull * x.T * x.H;
+    d.part = (float*)(d.mid3 + 3ull * x.T * x.DI);
+    hipLaunchKernelGGL(dnorm_kernel, dim3(x.T), dim3(kThreads), 0, s, d);
+    DenseArgs du = d;
+    du.S = 1u;
+    const uint32_t nb = (uint32_t)cd(cd(x.T, np), kRB);
+#define WL_DENSE(NB)                                                              \
+    case NB:                                                                      \
+        hipLaunchKernelGGL((dgemm_kernel<true, NB>), dim3(n_cu), dim3(kGT), 0, s, du); \
+        hipLaunchKernelGGL((dgemm_kernel<false, NB>), dim3(n_cu), dim3(kGT), 0, s, d); \
+        break
+    switch (nb) {
+        WL_DENSE(1);
+        WL_DENSE(2);
+        WL_DENSE(3);
+        WL_DENSE(4);
+    }
+#undef WL_DENSE
+    hipLaunchKernelGGL(dsum_kernel, dim3((uint32_t)(((uint64_t)x.T * x.H / 4u + 255u) / 256u)), dim3(256), 0, s, d);
     return (int)hipGetLastError();
 }
 
