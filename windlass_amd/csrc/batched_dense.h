@@ -52,13 +52,13 @@ __global__ void __launch_bounds__(kThreads) dnorm_kernel(const DenseArgs d) {
 // blocks) x 8 waves x two tiles of 16 weight rows x one of the S splits of K. UP:
 // tile 0 gate rows, tile 1 the same up rows, K = H, S = 1, SwiGLU values as pieces
 // to mid3. Down: 32 output rows per wave, K = DI, f32 partial rows. A step is 128
-// columns; a load takes 64 bytes of each of 16 rows (lane (n, g): row n, columns
-// 32 k + 8 g of the step). Columns past K and rows past the matrix are out of
+// columns; a load takes 128 bytes, a cache line, of each of eight rows, and the
+// lanes trade halves (rows_swap; 64 bytes of each of 16 rows: 1 % slower at 200
+// positions, 4 % at 8 of hidden 2944, inter 6832). Columns past K and rows past the matrix are out of
 // range: zeros on both sides. The slot is SharedK's. Bound by the LDS reads of
 // the fragments and the matrix cores (each near 3100 cycles of a step with four
 // row blocks) and, measured, the weight loads: 200 positions of hidden 6144, inter
-// 12288 take 268 us gate/up and 138 us down under a kernel trace, the call 377 us;
-// one position at a time it took 15200.
+// 12288 take 372 us (two thirds gate/up); one position at a time they took 15200.
 template <bool UP, uint32_t NB>
 struct DenseK {
     using AS = AStreamS;
@@ -110,9 +110,21 @@ struct DenseK {
         const uint32_t h = j % kRB2, pc = j / kRB2, cg = n ^ ((4u * v + g) & 15u), c = col0 + 128u * s;
         dma16<S>(A.rs, (16u * pc + 8u * h + v) * 1024u, c + 8u * cg < K ? A.base[h] : kOOBV, 2u * c + pc * A.kd2);
     }
+    // Loads 2i and 2i + 1 of a tile: its first and last eight rows, 64 columns.
     WL_MEM void load(uint32_t s, WB& W, uint32_t j) const {
-        const uint32_t t = j / 4u, k = j % 4u, c = col0 + 128u * s + 32u * k;
-        W.w[j] = bld16(make_rsrc(t ? w1 : w0, wbytes), c + 8u * g < K ? vw[t] : kOOBV, 2u * c);
+        const uint32_t t = j / 4u, c = col0 + 128u * s + 64u * (j % 4u / 2u);
+        W.w[j] = bld16(make_rsrc(t ? w1 : w0, wbytes), c + 8u * g + 4u * (n & 8u) < K ? vw[t] + (j % 2u) * 16u * K : kOOBV,
+                       2u * c);
+    }
+    // Such a pair -> row n of the tile in lane (n, g): columns 8 g of its first 32
+    // in x, of its last 32 in y (lanes n >= 8 of x trade with lanes n < 8 of y).
+    WL_MEM static void rows_swap(u32x4& x, u32x4& y) {
+#pragma unroll
+        for (uint32_t q = 0; q < 4; q++) {
+            const int a = (int)x[q], b = (int)y[q];
+            x[q] = (uint32_t)__builtin_amdgcn_update_dpp(a, b, 0x128, 0xF, 0xC, false);  // row_ror:8, lanes 8-15
+            y[q] = (uint32_t)__builtin_amdgcn_update_dpp(b, a, 0x128, 0xF, 0x3, false);  // lanes 0-7
+        }
     }
     WL_MEM void begin(uint32_t i) {
         cu = unit(i);
@@ -121,21 +133,28 @@ struct DenseK {
 #pragma unroll
             for (uint32_t m = 0; m < NB; m++) sum[t][m] = err[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    // (SharedK::comp's order)
+    // Iteration it: columns 32 (it % 4) of the step, of the third pieces, then the
+    // second, then the first: the sums round at the small pieces' size until the
+    // last four (error against 64 bits 9.9e-8 at 200 positions; 1.4e-7 in
+    // SharedK::comp's order, where all twelve round at the first piece's).
     template <class Next>
     WL_MEM void comp(uint32_t, const uint8_t* sl, WB& W, Next next) {
         auto frag = [&](uint32_t it, uint32_t m) {
-            return as_bf16x8(*(const u32x4*)(sl + ((it % 3u) * 64u + m * 16u) * 256u + (lob ^ (64u * (it / 3u)))));
+            return as_bf16x8(*(const u32x4*)(sl + ((2u - it / 4u) * 64u + m * 16u) * 256u + (lob ^ (64u * (it % 4u)))));
         };
         bf16x8 af[2][NB];
 #pragma unroll
         for (uint32_t m = 0; m < NB; m++) af[0][m] = frag(0u, m);
 #pragma unroll
         for (uint32_t it = 0; it < 12u; it++) {
-            const uint32_t k = it / 3u;
+            const uint32_t k = it % 4u;
             if (it + 1u < 12u) {
 #pragma unroll
                 for (uint32_t m = 0; m < NB; m++) af[(it + 1u) & 1u][m] = frag(it + 1u, m);
+            }
+            if (it == 0u || it == 2u) {
+                rows_swap(W.w[k], W.w[k + 1u]);
+                rows_swap(W.w[4u + k], W.w[5u + k]);
             }
             next(it, 12u);
 #pragma unroll
@@ -202,7 +221,7 @@ __global__ void __launch_bounds__(kGT) dgemm_kernel(const DenseArgs d) {
     k.v = uni(threadIdx.x >> 6);
 #pragma unroll
     for (uint32_t t = 0; t < 2; t++)
-        k.vw[t] = ((UP ? 16u * k.v : 32u * k.v + 16u * t) + k.n) * k.K * 2u + 16u * k.g;
+        k.vw[t] = ((UP ? 16u * k.v : 32u * k.v + 16u * t) + (k.n & 7u)) * k.K * 2u + 16u * k.g + 8u * (k.n & 8u);
     k.lob = k.n * 256u + 16u * (k.g ^ k.n);
     run_units(k);
 }
