@@ -364,21 +364,34 @@ WL_DEV f32x4 mmq(u32x4 w, i32x8 x, f32x4 c, uint32_t ow, uint32_t sw, uint32_t o
 #undef WL_MMQ
     return c;
 }
-// Piece p of a staged k tile of 16 rows at `tile`; lo8: the lane's offset of
-// its 8-byte parts.
+// A staged k tile of 16 rows: kilobyte 2 u + h holds units 8 u .. 8 u + 7 of rows
+// 8 h .. 8 h + 7, 128 bytes a row, unit c in its 16-byte place c ^ q_swizzle(row),
+// so that the 16 rows of a fragment read fall in different banks.
+WL_DEV uint32_t q_swizzle(uint32_t n) { return (n & 7u) ^ (n >> 3); }
+// The lane's offsets of unit g of row n, and of its 8 bytes of unit g / 2.
+WL_DEV uint32_t q_lo16() {
+    const uint32_t lane = threadIdx.x & 63u, n = lane & 15u, g = lane >> 4;
+    return 1024u * (n >> 3) + 128u * (n & 7u) + 16u * (g ^ q_swizzle(n));
+}
 WL_DEV uint32_t q_lo8() {
     const uint32_t lane = threadIdx.x & 63u, n = lane & 15u, g = lane >> 4;
-    return 256u * (g >> 1) + 16u * n + 8u * (g & 1u);
+    return 1024u * (n >> 3) + 128u * (n & 7u) + 16u * ((g >> 1) ^ q_swizzle(n)) + 8u * (g & 1u);
 }
+// From the lane's offset lo of unit i (< 4 for c a multiple of 4, < 2 for an even
+// c): that of unit c + i.
+WL_DEV const uint8_t* q_at(const uint8_t* tile, uint32_t c, uint32_t lo) {
+    return tile + 2048u * (c / 8u) + (lo ^ (16u * (c % 8u)));
+}
+// Piece p of the tile.
 template <uint32_t P>
-WL_DEV i32x8 q_frag(const uint8_t* tile, uint32_t p, uint32_t lane16, uint32_t lo8) {
-    const u32x4 h = *(const u32x4*)(tile + 1024u * p + lane16);
-    const u32x2 l = *(const u32x2*)(tile + 1024u * P + 512u * p + lo8);
+WL_DEV i32x8 q_frag(const uint8_t* tile, uint32_t p, uint32_t lo16, uint32_t lo8) {
+    const u32x4 h = *(const u32x4*)q_at(tile, 4u * p, lo16);
+    const u32x2 l = *(const u32x2*)q_at(tile, 4u * P + 2u * p, lo8);
     return i32x8{(int)h.x, (int)h.y, (int)h.z, (int)h.w, (int)l.x, (int)l.y, 0, 0};
 }
 template <uint32_t P>
 WL_DEV u32x2 q_scales(const uint8_t* tile, uint32_t lo8) {
-    return *(const u32x2*)(tile + 1536u * P + lo8);
+    return *(const u32x2*)q_at(tile, 6u * P, lo8);
 }
 // Two chunks of 64 columns of a row pair (lane (n, g): row 32 q + n + 16 (g >>
 // 1), block g & 1) -> 128 columns of each of its halves, in place.
@@ -393,11 +406,13 @@ WL_DEV void pair_swap(u32x4& x, u32x4& y) {
 }
 
 // MB row blocks, KT k tiles per step: the slot holds tile (q, m), number MB q + m.
-// A DMA of a tile fills units c = 4u .. 4u + 3 of its 16 rows: lane (n, g) reads
-// 16 bytes of row 16 m + n, at its base + 64 u. Wave v takes u = v of every tile;
-// of a record of ten such groups, the two left over of four tiles at once: wave
-// v group 8 + v % 2 of tile 4 x + v / 2 (past the tiles: out of range, into the
-// slot's end). Absent rows, k tiles past the row's end and units past the record
+// A DMA of a tile fills one of its kilobytes: 128 bytes of each of eight rows, a
+// row by eight lanes next to each other (lane l: row 8 h + l / 8). Wave v takes
+// kilobyte v of every tile; of a record of ten, the two left over of four tiles at
+// once: wave v kilobyte 8 + v % 2 of tile 4 x + v / 2 (past the tiles: out of
+// range, into the slot's end). (Lanes that took 64 bytes of each of 16 rows, every
+// quarter wave 16 cache lines: 1000 tokens 1588 us a call, now 1556; 333 of hidden
+// 2944 309, 305; 7, 64 and 4096 the same within 0.4 %.) Absent rows, k tiles past the row's end and units past the record
 // land as zeros (zero scales too: their products are zero).
 template <uint32_t MB>
 struct AStreamQ {
@@ -421,13 +436,13 @@ struct QBase {
     static_assert(kTileB * kTiles + (kLeft ? 8192u : 0u) <= kSlotB, "a step's tiles fit a slot");
     const DecodeArgs& a;
     const BatchArgs& b;
-    uint32_t H, I, E, K, nk, S, nq, parts, nst, nst2, nu, v, lane, g, uoff;
+    uint32_t H, I, E, K, nk, S, nq, parts, nst, nst2, nu, v, lane, uoff;
     PassTab pt;
     const uint8_t* const* stab;
     NativeLayout NL;
     Cursor cn, cc;  // positions of the loads and of the compute
     const uint8_t* wbase;  // the weight stream's block and size (see SharedK)
-    uint32_t wbytes, wpart, vw, vs, lo8;
+    uint32_t wbytes, wpart, vw, vs, lo8, lo16;
     UnitInfo cu, un;     // the unit computed, the unit whose loads go out
     const uint16_t *tt, *ent;  // UP: the token table; the entries where this kernel grouped them (or null)
 
@@ -450,7 +465,7 @@ struct QBase {
         wbase = blk;
         wbytes = blk ? (uint32_t)NL.total : 0u;
         wpart = x.part;
-        const uint32_t kd = UP ? H : I, n = lane & 15u;
+        const uint32_t kd = UP ? H : I, n = 8u * (v & 1u) + lane / 8u, c8 = lane % 8u ^ q_swizzle(n);
         const uint32_t nrow = UP ? b.T : b.T * (K + ((b.flags & kBatchShared4) ? 1u : 0u));
         const uint32_t rowb = (uint32_t)q6_row_bytes(P, kd);
         A.rs = make_rsrc(x.live ? (UP ? (const uint8_t*)b.norm : b.mid6) : nullptr, x.live ? nrow * rowb : 0u);
@@ -459,16 +474,16 @@ struct QBase {
             const uint32_t r = kRB * m + n;
             uint32_t row = x.row0 + r;
             if (UP) row = x.e == a.E ? row - b.T * K : x.live ? table_token(tt, b.tcap, kRB * NB, i, r, x.nt) : 0u;
-            return r < x.nt ? row * rowb + 16u * g : kOOBV;
+            return r < x.nt ? row * rowb + 16u * c8 : kOOBV;
         };
 #pragma unroll
         for (uint32_t m = 0; m < NB; m++) {
             const uint32_t o = row_at(m);
-            A.base[m] = o == kOOBV ? o : o + 64u * v;
+            A.base[m] = o == kOOBV ? o : o + 128u * (v / 2u);
         }
         if (kLeft) {
-            const uint32_t c = 4u * (8u + v % 2u) + g, o = row_at(v / 2u % NB);
-            A.left = v / 2u < kTiles && c < q6_units(P) && o != kOOBV ? o + 64u * (8u + v % 2u) : kOOBV;
+            const uint32_t o = row_at(v / 2u % NB);
+            A.left = v / 2u < kTiles && 32u + c8 < q6_units(P) && o != kOOBV ? o + 512u : kOOBV;
         }
     }
     template <int SL>
@@ -551,11 +566,11 @@ struct QNarrow : QBase<UP, NB, 2> {
         i32x8 af[AH + 1u];
         u32x2 sa[NB];
         uint32_t sx = 0u, sy = 0u;
-        const uint32_t lane16 = 16u * this->lane;
+        const uint32_t lo16 = this->lo16;
         auto tile = [&](uint32_t q, uint32_t m) { return sl + (q * NB + m) * QB::kTileB; };
         auto frag = [&](uint32_t it) {
             const uint32_t m = it % NB, p = it / NB % P, q = it / (NB * P);
-            return q_frag<P>(tile(q, m), p, lane16, this->lo8);
+            return q_frag<P>(tile(q, m), p, lo16, this->lo8);
         };
 #pragma unroll
         for (uint32_t it = 0; it < AH; it++) af[it] = frag(it);
@@ -648,8 +663,8 @@ struct QWide : QBase<UP, NB, 1> {
         constexpr uint32_t N = P * NB, AH = 2u;
         i32x8 af[AH + 1u];
         u32x2 sa[NB];
-        const uint32_t lane16 = 16u * this->lane;
-        auto frag = [&](uint32_t it) { return q_frag<P>(sl + (it % NB) * QB::kTileB, it / NB, lane16, this->lo8); };
+        const uint32_t lo16 = this->lo16;
+        auto frag = [&](uint32_t it) { return q_frag<P>(sl + (it % NB) * QB::kTileB, it / NB, lo16, this->lo8); };
 #pragma unroll
         for (uint32_t it = 0; it < AH; it++) af[it] = frag(it);
 #pragma unroll
@@ -800,9 +815,9 @@ WL_DEV uint32_t run_routed(const DecodeArgs& a, const BatchArgs& b, uint32_t E, 
     const uint32_t U = pt.n * w.parts, b0 = (blockIdx.x + gridDim.x - w.uoff) % gridDim.x;
     w.nu = U > b0 ? cdiv(U - b0, gridDim.x) : 0u;
     w.lane = threadIdx.x & 63u;
-    w.g = w.lane >> 4;
     w.v = uni(threadIdx.x >> 6);
     w.lo8 = q_lo8();
+    w.lo16 = q_lo16();
     w.pt = pt;
     w.stab = stab;
     w.NL = NativeLayout::make(H, I);
@@ -821,9 +836,9 @@ WL_DEV uint32_t run_routed(const DecodeArgs& a, const BatchArgs& b, uint32_t E, 
 // Routed rows as fp6 pieces against fp4 weights run at 3.5 times the rate of bf16
 // pieces and need no conversion of the weights. Whole calls, hidden 6144, inter
 // 2048, 8 of 256 experts (256 work-groups of eight waves), before (bf16 pieces,
-// passes of 32 and 64) and now: 4096 tokens 8440 and 4940 us, 1000 tokens 2310 and
-// 1585, 64 tokens (one row block per expert; the weights' 4.4 GB at 6 TB/s) 724 and
-// 739, 7 tokens 213.0 and 214.4; hidden 2944, inter 1408, 6 of 160 experts, 333 tokens: 457 and 310.
+// passes of 32 and 64) and now: 4096 tokens 8360 and 4900 us, 1000 tokens 2307 and
+// 1556, 64 tokens (one row block per expert; the weights' 4.4 GB at 6 TB/s) 751 and
+// 757, 7 tokens 215.7 and 218.1; hidden 2944, inter 1408, 6 of 160 experts, 333 tokens: 462 and 305.
 // Error against 64 bits: 8.1e-7 and 4.5e-7 at 4096 tokens, 3.5e-7 and 1.5e-7 at 64.
 template <bool UP>
 WL_DEV void run_gemm(const DecodeArgs* pa, const BatchArgs& b) {

@@ -1,5 +1,5 @@
 // q6.h — f32 rows in five 6-bit floating-point pieces, the operands of the
-// routed experts' GEMMs on gfx950's scaled matrix instruction (batched_q6.h).
+// routed experts' GEMMs on gfx950's scaled matrix instruction (batched_gemm.h).
 //
 // v_mfma_scale_f32_16x16x128_f8f6f4 takes the MXFP4 weights as they lie in the
 // native block (a lane's 16 bytes are its 32 values, its E8M0 byte the scale
@@ -27,8 +27,7 @@
 // 4p + g the first 16 bytes of piece p of block g, c = 4P + 2p + h the last 8
 // bytes of piece p of blocks 2h and 2h + 1, c = 6P + h the scale bytes (8 per
 // block, P used) of blocks 2h and 2h + 1: 512 bytes for five pieces, 608 for
-// six. DMA'd into LDS as [unit c][row n] (16 rows), every read of an A operand
-// is one contiguous kilobyte, half kilobyte or its 8-byte scales over the wave.
+// six. A DMA into LDS takes eight units of each of eight rows.
 #pragma once
 #include "dev_common.h"
 
