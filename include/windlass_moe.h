@@ -121,10 +121,12 @@ wl_status wl_set_layer_mxfp4(wl_ctx* ctx, uint32_t layer, const uint16_t* d_rout
  * caller-owned, 16-byte aligned, valid while the layer is run. wl_run_moe on
  * the layer writes down(silu(gate x) * up x), x = RMSNorm(d_hidden), without
  * the residual (two GEMV launches, no host round trip); wl_run_moe_residual,
- * wl_run_chain and wl_run_moe_batched (one position at a time, as the
- * reference's layer-major prefill does for these layers, :985-994) add the
- * residual. The norm tap holds x. Synchronises the device. dense_inter: a
- * multiple of 8, at most 16384. */
+ * wl_run_chain and wl_run_moe_batched (up to 512 positions at once; the
+ * reference's layer-major prefill runs these layers one position at a time,
+ * :985-994) add the residual. The norm tap holds x. Synchronises the device.
+ * dense_inter: a multiple of 8, at most 16384. The context then holds a scratch
+ * for calls of many positions (170 MB at hidden 6144, inter 12288); where there
+ * is no memory for it those calls run one position at a time. */
 wl_status wl_set_layer_dense(wl_ctx* ctx, uint32_t layer, const uint16_t* d_post_ln, const uint16_t* d_gate,
                              const uint16_t* d_up, const uint16_t* d_down, uint32_t dense_inter);
 
@@ -256,7 +258,9 @@ wl_status wl_run_chain(wl_ctx* ctx, uint32_t first_layer, uint32_t n_layers, flo
  * At most 816 routed experts (the GEMM kernels keep the expert tables in LDS
  * beside the activation slots); a wider config fails with WL_ERR_INVALID.
  * Scratch grows to the largest chunk seen (context-owned; growing
- * synchronises the device). */
+ * synchronises the device). A dense layer's call uses the scratch made when the
+ * layer was bound; a row agrees with the row of a call of another length, or with
+ * wl_run_moe_residual's, within rounding, not bit for bit. */
 wl_status wl_run_moe_batched(wl_ctx* ctx, uint32_t layer, uint32_t n_tokens, const float* d_hidden,
                              const float* d_resid, float* d_out, void* stream);
 
@@ -267,7 +271,8 @@ wl_status wl_run_moe_batched(wl_ctx* ctx, uint32_t layer, uint32_t n_tokens, con
  * but the scratch comes from a static 64 MiB device array of the library
  * (one per GPU, held until the process ends) instead of context memory that
  * wl_run_moe_batched grows on demand, so the call performs no hipMalloc,
- * hipFree or other allocation. Tokens run in chunks of as many as the array
+ * hipFree or other allocation (a dense layer's call is wl_run_moe_batched's,
+ * which makes none). Tokens run in chunks of as many as the array
  * holds (169 at hidden 6144 / inter 2048 / 8 of 256 experts); a shape whose
  * single token does not fit returns WL_ERR_INVALID. Every call on one GPU
  * shares that GPU's array, which keeps the last call's contents: calls that

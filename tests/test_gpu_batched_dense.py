@@ -17,6 +17,7 @@ from oracle import attention as A
 from oracle import moe_oracle as O
 from oracle import synth
 from windlass_amd import hip as H_, moe, synthdata
+from windlass_amd.model import DeviceModel
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-5
@@ -47,4 +48,84 @@ def test_dense_batched(gpu, T, shape):
         for t in (0, T // 2, T - 1):
             ctx.run_moe_batched(0, 1, d.ptr + 4 * H * t, None, one.ptr)
             assert O.rel_to_scale(one.download(np.float32), got[t]) < TOL, t
+    ctx.close()
+
+
+def _dense(ctx, layer, H, DI, seed, ln=True):
+    """Binds synthetic dense weights; the buffers, to be kept."""
+    w = synthdata.dense_mlp(H, DI, seed, layer)
+    dev = {k: H_.DeviceBuffer.from_array(v) for k, v in w.items()}
+    ctx.set_layer_dense(layer, dev["post_ln"].ptr if ln else None, dev["gate"].ptr, dev["up"].ptr, dev["down"].ptr, DI)
+    return dev
+
+
+def _rows(H, T, seed):
+    return np.stack([synth.hidden_state(H, seed, t) for t in range(T)]).astype(np.float32)
+
+
+def test_dense_calls_keep_the_batched_routing_and_allocate_nothing(gpu):
+    """A dense call through either entry point leaves what the last MoE call of
+    that entry point can still be asked for (its counts, ids, weights and logits),
+    and takes no device memory: its scratch comes with the layer. A larger layer
+    bound later, a smaller one and a layer without a norm weight run the same way."""
+    c = dict(hidden=384, moe_inter=256, n_routed_experts=48, n_experts_per_tok=6, n_shared=1, routed_scaling=2.5,
+             rms_eps=1e-5)
+    H, T = c["hidden"], 70
+    dm = DeviceModel(c, seed=24, n_layers=4)  # layers 1 to 3 bound again below
+    keep = [_dense(dm.ctx, 1, H, 1096, 33), _dense(dm.ctx, 2, H, 264, 34), _dense(dm.ctx, 3, H, 2200, 35, ln=False)]
+    x = H_.DeviceBuffer.from_array(_rows(H, T, 3300))
+    o = H_.DeviceBuffer(4 * T * H)
+    for run in (dm.ctx.run_moe_batched, dm.ctx.run_moe_batched_noalloc):
+        run(0, T, x.ptr, None, o.ptr)
+        dm.ctx.check_error()
+        before = (dm.ctx.batched_counts(), *dm.ctx.batched_routing(T))
+        free0, _ = H_.mem_info()
+        for layer in (1, 2, 3):
+            run(layer, T, x.ptr, None, o.ptr)
+            H_.synchronize()
+        assert H_.mem_info()[0] == free0
+        after = (dm.ctx.batched_counts(), *dm.ctx.batched_routing(T))
+        assert before[0].sum() == T * c["n_experts_per_tok"]
+        for a, b in zip(before, after):
+            assert np.array_equal(a, b)
+    w = {k: synthdata.as_f32(synthdata.dense_mlp(H, 2200, 35, 3))[k] for k in ("gate", "up", "down")}
+    ref = A.dense_mlp(_rows(H, T, 3300), dict(w, post_ln=np.ones(H, np.float32)), dict(rms_eps=1e-5))
+    got, hs = o.download(np.float32).reshape(T, H), _rows(H, T, 3300)
+    for t in range(T):
+        assert O.rel_to_scale(ref[t] - hs[t], got[t]) < TOL, t
+    del keep
+    dm.close()
+
+
+def test_both_entry_points_and_graphs_give_the_same_bits(gpu):
+    """One call of 513 positions (a chunk of 512 and one more) through either entry
+    point, and captured into a graph through either and replayed three times with
+    eager work of the program between the replays: the same bits."""
+    H, DI, T = 3072, 1024, 513
+    ctx = moe.Context(moe.make_config(hidden=H, moe_inter=256, n_routed_experts=16, n_experts_per_tok=1, rms_eps=1e-5))
+    keep = _dense(ctx, 0, H, DI, 36)
+    x = H_.DeviceBuffer.from_array(_rows(H, T, 3600))
+    o = H_.DeviceBuffer(4 * T * H)
+    other = H_.DeviceBuffer(4 * 9 * H)
+    ctx.run_moe_batched(0, T, x.ptr, x.ptr, o.ptr)
+    eager = o.download(np.uint32)
+    st = H_.Stream()
+    for run in (ctx.run_moe_batched, ctx.run_moe_batched_noalloc):
+        o.zero()
+        run(0, T, x.ptr, x.ptr, o.ptr)
+        assert np.array_equal(o.download(np.uint32), eager)
+        g = H_.Graph(st)
+        g.begin()
+        run(0, T, x.ptr, x.ptr, o.ptr, st.handle)
+        g.end()
+        for rep in range(3):
+            o.zero()
+            H_.synchronize()
+            g.launch()
+            st.synchronize()
+            assert np.array_equal(o.download(np.uint32), eager), rep
+            run(0, 9, x.ptr, None, other.ptr, st.handle)
+            st.synchronize()
+        g.destroy()
+    del keep
     ctx.close()

@@ -161,7 +161,7 @@ struct wl_ctx {
     // norm weight [H] bf16 for a layer bound without one
     float *dense_g = nullptr, *dense_u = nullptr;
     uint32_t dense_cap = 0;
-    void* dense_buf = nullptr;  // batched scratch (dense_reserve)
+    void* dense_buf = nullptr;  // batched scratch (wl_set_layer_dense)
     size_t dense_bytes = 0;
     uint16_t* ones_ln = nullptr;
 };
@@ -435,7 +435,6 @@ void wl_destroy(wl_ctx* c) {
         delete C.lru;
     }
     if (c->batch.buf) (void)hipFree(c->batch.buf);
-    if (c->dense_buf) (void)hipFree(c->dense_buf);
     if (c->stage) (void)hipFree(c->stage);
     for (LayerState& L : c->layers)
         for (void* p : L.owned) (void)hipFree(p);
@@ -531,6 +530,9 @@ wl_status wl_set_layer_mxfp4(wl_ctx* c, uint32_t layer, const uint16_t* d_router
     return set_layer(c, layer, d_router_w, d_router_bias, d_post_attn_ln, nullptr, parts);
 }
 
+// Positions of a dense layer run at once.
+constexpr uint32_t kDenseChunk = 512;
+
 wl_status wl_set_layer_dense(wl_ctx* c, uint32_t layer, const uint16_t* d_post_ln, const uint16_t* d_gate,
                              const uint16_t* d_up, const uint16_t* d_down, uint32_t dense_inter) {
     if (!c) return WL_ERR_INVALID;
@@ -551,6 +553,24 @@ wl_status wl_set_layer_dense(wl_ctx* c, uint32_t layer, const uint16_t* d_post_l
             (st = dalloc(c, &c->dense_u, 4 * (size_t)dense_inter)) != WL_OK)
             return st;  // a smaller pair stays owned by the context until it is destroyed
         c->dense_cap = dense_inter;
+    }
+    // The scratch of calls over many positions: made here, so that those calls
+    // neither allocate nor synchronise. A graph may hold it, so one that is too
+    // small stays until the context goes; sizes are those of powers of two, all of
+    // them together less than twice the largest. Without memory for it positions
+    // run one at a time.
+    uint32_t pow2 = 8;
+    while (pow2 < dense_inter) pow2 *= 2u;
+    const size_t bytes = kDenseChunk * wl::dense_token_bytes(H, pow2);
+    if (bytes > c->dense_bytes) {
+        void* p = nullptr;
+        if (hipMalloc(&p, bytes) == hipSuccess) {
+            c->allocs.push_back(p);
+            c->dense_buf = p;
+            c->dense_bytes = bytes;
+        } else {
+            (void)hipGetLastError();
+        }
     }
     if (!d_post_ln && !c->ones_ln) {
         wl_status st = dalloc(c, &c->ones_ln, 2 * (size_t)H);
@@ -1285,33 +1305,18 @@ static wl_status batched_run(wl_ctx* c, uint32_t layer, uint32_t n_tokens, const
     return WL_OK;
 }
 
-// A dense layer of a batched call: the dense MLP per position (the reference
-// has nothing to amortise there either and runs run_moe + residual_add per
-// position, src/glm_layer_runner.cuh:985-994). No scratch beyond the layer's.
-// The dense layers' batched scratch, of its own: the batched taps read the other
-// after a dense call. False: no memory for it (nothing lost).
-static bool dense_reserve(wl_ctx* c, size_t bytes) {
-    if (bytes <= c->dense_bytes) return true;
-    void* p = nullptr;
-    // (launches in flight may still use the old one)
-    if (hipDeviceSynchronize() != hipSuccess || hipMalloc(&p, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    if (c->dense_buf) (void)hipFree(c->dense_buf);
-    c->dense_buf = p;
-    c->dense_bytes = bytes;
-    return true;
-}
-// Positions of a dense layer in chunks through the batched kernels; `scratch`
-// holds `chunk` positions. A chunk of one position takes the decode kernels (all
-// of them where there is no scratch for two).
+// A dense layer of a batched call (the reference runs run_moe + residual_add per
+// position, src/glm_layer_runner.cuh:985-994): chunks of positions through the
+// batched kernels on the context's dense scratch, under capture too. A chunk of
+// one position takes the decode kernels, as all do where there is no scratch.
 static wl_status batched_dense(wl_ctx* c, uint32_t layer, uint32_t n_tokens, const float* d_hidden,
-                               const float* d_resid, float* d_out, void* scratch, uint64_t chunk, void* stream) {
+                               const float* d_resid, float* d_out, void* stream) {
     const size_t H = c->cfg.hidden;
     const LayerState& L = c->layers[layer];
+    const uint64_t fit = c->dense_bytes / wl::dense_token_bytes(c->cfg.hidden, L.dense_inter);
+    const uint32_t chunk = (uint32_t)std::max<uint64_t>(1u, std::min<uint64_t>(kDenseChunk, fit));
     for (uint32_t t = 0; t < n_tokens;) {
-        const uint32_t n = (uint32_t)std::min<uint64_t>(n_tokens - t, std::max<uint64_t>(chunk, 1u));
+        const uint32_t n = std::min(n_tokens - t, chunk);
         const float *x = d_hidden + t * H, *add = d_resid ? d_resid + t * H : nullptr;
         float* y = d_out + t * H;
         t += n;
@@ -1322,7 +1327,7 @@ static wl_status batched_dense(wl_ctx* c, uint32_t layer, uint32_t n_tokens, con
         }
         const wl::DenseBatch m{x, add, y, L.ln, L.mlp_gate, L.mlp_up, L.mlp_down, n, c->cfg.hidden, L.dense_inter,
                                c->cfg.rms_eps, t == n_tokens ? c->norm : nullptr};
-        const int e = wl::launch_dense_batched(m, (uint32_t)c->n_cu, scratch, stream);
+        const int e = wl::launch_dense_batched(m, (uint32_t)c->n_cu, c->dense_buf, stream);
         if (e != 0) return hip_fail(c, (hipError_t)e, "batched dense MLP launch");
     }
     return WL_OK;
@@ -1333,16 +1338,7 @@ wl_status wl_run_moe_batched(wl_ctx* c, uint32_t layer, uint32_t n_tokens, const
     if (!c) return WL_ERR_INVALID;
     wl_status s = batched_check(c, layer, n_tokens, d_hidden, d_resid, d_out);
     if (s != WL_OK) return s;
-    if (c->layers[layer].dense) {
-        // (a stream under capture: no scratch that may grow later under the graph)
-        constexpr uint32_t kDenseChunk = 512;
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        const uint64_t chunk = std::min(n_tokens, kDenseChunk);
-        const bool ok = chunk > 1 && hipStreamIsCapturing((hipStream_t)stream, &cs) == hipSuccess &&
-                        cs == hipStreamCaptureStatusNone &&
-                        dense_reserve(c, chunk * wl::dense_token_bytes(c->cfg.hidden, c->layers[layer].dense_inter));
-        return batched_dense(c, layer, n_tokens, d_hidden, d_resid, d_out, c->dense_buf, ok ? chunk : 1u, stream);
-    }
+    if (c->layers[layer].dense) return batched_dense(c, layer, n_tokens, d_hidden, d_resid, d_out, stream);
     // Tokens run in chunks: bounded scratch, and every piece array stays under
     // 2 GB.
     const uint32_t chunk = batch_offset_cap(c);
@@ -1356,11 +1352,7 @@ wl_status wl_run_moe_batched_noalloc(wl_ctx* c, uint32_t layer, uint32_t n_token
     if (!c) return WL_ERR_INVALID;
     wl_status s = batched_check(c, layer, n_tokens, d_hidden, d_resid, d_out);
     if (s != WL_OK) return s;
-    if (c->layers[layer].dense) {
-        const uint64_t chunk =
-            c->scratch ? wl::noalloc_scratch_bytes() / wl::dense_token_bytes(c->cfg.hidden, c->layers[layer].dense_inter) : 0u;
-        return batched_dense(c, layer, n_tokens, d_hidden, d_resid, d_out, c->scratch, chunk, stream);
-    }
+    if (c->layers[layer].dense) return batched_dense(c, layer, n_tokens, d_hidden, d_resid, d_out, stream);
     if (c->n_bound[layer] == 0) {
         // a source-backed layer reads its routing back on the host (a
         // synchronisation), which a stream under capture does not allow
