@@ -129,3 +129,47 @@ def test_both_entry_points_and_graphs_give_the_same_bits(gpu):
         g.destroy()
     del keep
     ctx.close()
+
+
+def test_values_past_bf16_range(gpu):
+    """SwiGLU values that leave the f32 range, or lie between bf16's largest value
+    and f32's: the same infinities, NaNs and finite values as one position at a
+    time. Planted inner rows: 5 the product of 2^65 and 2^65 (infinite; 0 for a
+    negative input), 70 the product 2^127 * 1.998. Down weighs the first with 0 in
+    some rows (NaN) and the second with 2^-20."""
+    H, DI, T = 384, 264, 20
+    ctx = moe.Context(moe.make_config(hidden=H, moe_inter=256, n_routed_experts=16, n_experts_per_tok=1, rms_eps=1e-5))
+    w = synthdata.dense_mlp(H, DI, 37, 0)
+
+    def bits(x):
+        return (np.asarray(x, np.float32).view(np.uint32) >> 16).astype(np.uint16)
+
+    for m in ("gate", "up"):
+        w[m][[5, 70]] = 0
+    w["gate"][5, 7] = w["up"][5, 7] = bits(2.0**65)
+    w["gate"][70, 9] = bits(2.0**64)
+    w["up"][70, 9], w["up"][70, 11] = bits(2.0**63 * 1.9921875), bits(2.0**63 * 1.5 / 256)
+    w["down"][:, 5] = bits(1.0)
+    w["down"][::3, 5] = 0
+    w["down"][1::7, 5] = bits(-1.0)
+    w["down"][:, 70] = bits(2.0**-20)
+    w["post_ln"][:] = bits(1.0)
+    dev = {k: H_.DeviceBuffer.from_array(v) for k, v in w.items()}
+    ctx.set_layer_dense(0, dev["post_ln"].ptr, dev["gate"].ptr, dev["up"].ptr, dev["down"].ptr, DI)
+    hs = np.ones((T, H), np.float32)  # normalised: 1 - 5e-6
+    hs[1::2, 7] = -1.0  # these rows stay finite
+    x = H_.DeviceBuffer.from_array(hs)
+    o, one = H_.DeviceBuffer(4 * T * H), H_.DeviceBuffer(4 * H)
+    ctx.run_moe_batched(0, T, x.ptr, None, o.ptr)
+    got = o.download(np.float32).reshape(T, H)
+    for t in range(T):
+        ctx.run_moe_batched(0, 1, x.ptr + 4 * H * t, None, one.ptr)
+        ref = one.download(np.float32)
+        fin = np.isfinite(ref)
+        assert np.array_equal(np.isnan(ref), np.isnan(got[t])), t
+        assert np.array_equal(ref[np.isinf(ref)], got[t][np.isinf(ref)]), t
+        assert fin.all() if t % 2 else (not fin.any() and np.isinf(ref).any() and np.isnan(ref).any())
+        if fin.any():
+            assert np.abs(ref[fin]).min() > 2.0**106
+            assert O.rel_to_scale(ref[fin], got[t][fin]) < TOL, t
+    ctx.close()

@@ -193,7 +193,7 @@ struct DenseK {
                 float xs[4];
 #pragma unroll
                 for (uint32_t i = 0; i < 4; i++) xs[i] = silu_mul(total(0, m, i), total(1, m, i));
-                if (r < cu.nt && col < rows) store_pieces4(d.mid3 + (size_t)(cu.row0 + r) * 3u * rows + col, rows, xs);
+                if (r < cu.nt && col < rows) store_pieces4<true>(d.mid3 + (size_t)(cu.row0 + r) * 3u * rows + col, rows, xs);
                 __builtin_amdgcn_sched_barrier(0);
             } else {
 #pragma unroll

@@ -46,11 +46,27 @@ constexpr uint32_t kTB = 8;          // tokens per routing work-group
 constexpr uint32_t kGW = 8;         // waves of a GEMM work-group
 constexpr uint32_t kGT = 64 * kGW;  // its threads
 
-// The three bf16 pieces of 4 consecutive values at p, p + stride, p + 2 stride.
+// split3 of any value: one past bf16's largest starts with that (rounded to
+// infinity it would leave -infinity to the other pieces, and a NaN), an infinity
+// is its first piece alone.
+WL_DEV void split3_any(float x, uint32_t& h, uint32_t& m, uint32_t& l) {
+    const uint32_t u = __float_as_uint(x);
+    h = f2bf(x);
+    if ((h & 0x7FFFu) == 0x7F80u) h = u >> 16;
+    const float r1 = (u & 0x7FFFFFFFu) == 0x7F800000u ? 0.f : x - bf2f(h);
+    m = f2bf(r1);
+    l = f2bf(r1 - bf2f(m));
+}
+// The three bf16 pieces of 4 consecutive values at p, p + stride, p + 2 stride
+// (ANY: of values that may leave bf16's range).
+template <bool ANY = false>
 WL_DEV void store_pieces4(uint16_t* p, uint32_t stride, const float (&x)[4]) {
     uint32_t h[4], md[4], l[4];
 #pragma unroll
-    for (int q = 0; q < 4; q++) split3(x[q], h[q], md[q], l[q]);
+    for (int q = 0; q < 4; q++) {
+        if constexpr (ANY) split3_any(x[q], h[q], md[q], l[q]);
+        else split3(x[q], h[q], md[q], l[q]);
+    }
     auto pack = [](const uint32_t (&x)[4]) {
         return (uint64_t)(x[0] | (x[1] << 16)) | ((uint64_t)(x[2] | (x[3] << 16)) << 32);
     };
