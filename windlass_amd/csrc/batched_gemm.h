@@ -8,7 +8,7 @@
 // cycles of MFMA took 4576, the loads adding 112 cycles each). A pipeline runs
 // units of one form (a token pass of NB row blocks of 16 tokens times a block of
 // weight rows, in nst steps of K): the bf16 shared expert (SharedK), then the
-// routed passes from five row blocks down to one (QWide, QNarrow). A work-group
+// routed passes from four row blocks down to one (QWide, QNarrow). A work-group
 // walks its units u = blockIdx.x + G i of each pipeline. Activations arrive in
 // LDS by DMA (buffer_load ... lds), weights in registers. The weights are the
 // matrix instructions' A operand (its rows), the tokens its columns: a lane then
@@ -52,7 +52,8 @@ struct UnitInfo {
 };
 
 // ---- pipeline ------------------------------------------------------------------------
-// Position of a stream in the units' steps: my unit i, its step s.
+// Position of a stream in the units' steps: my unit i (of a pipeline whose units may
+// run their steps twice, that run), its step s.
 struct Cursor {
     uint32_t i, s;
 };
@@ -92,15 +93,14 @@ WL_DEV void unit_step(Kn& k, typename Kn::AS& A, typename Kn::WB& cur, typename 
     };
     __builtin_amdgcn_sched_barrier(0);
     k.comp(k.cc.s, slot<S>(), cur, next);
-    if (advance(k.cc, k.nst)) {
-        if (k.cc.i <= k.nu) k.finish();
+    if (advance(k.cc, k.nst) && k.unit_end()) {
+        if (k.cu.live) k.finish();
         k.begin(k.cc.i);
     }
 }
 template <class Kn>
 WL_DEV void run_units(Kn& k) {
     if (k.nu == 0u) return;
-    const uint32_t Z = k.nu * k.nst;
     typename Kn::AS A;
     typename Kn::WB B0, B1, B2;
     k.cn = k.cc = Cursor{0u, 0u};
@@ -116,11 +116,11 @@ WL_DEV void run_units(Kn& k) {
 #pragma unroll
     for (uint32_t j = 0; j < Kn::kLoads; j++) k.load(k.cn.s, B1, j);
 #pragma unroll 1
-    for (uint32_t z = 0; z < Z; z += 3u) {
+    do {
         unit_step<0>(k, A, B0, B2);
         unit_step<1>(k, A, B1, B0);
         unit_step<2>(k, A, B2, B1);
-    }
+    } while (k.cu.live);
 }
 
 // ---- outputs ---------------------------------------------------------------------------
@@ -185,6 +185,7 @@ struct SharedK {
     static constexpr bool kSum = NT == 1u;
     f32x4 acc[NT][NB][2], sum[kSum ? NT : 1][kSum ? NB : 1];
 
+    WL_MEM static bool unit_end() { return true; }  // the unit ends with its steps
     WL_MEM UnitInfo unit(uint32_t i) const {
         UnitInfo x{false, 0u, 0u, 0u, 0u};
         if (i >= nu) return x;
@@ -383,15 +384,13 @@ WL_DEV const uint8_t* q_at(const uint8_t* tile, uint32_t c, uint32_t lo) {
     return tile + 2048u * (c / 8u) + (lo ^ (16u * (c % 8u)));
 }
 // Piece p of the tile.
-template <uint32_t P>
 WL_DEV i32x8 q_frag(const uint8_t* tile, uint32_t p, uint32_t lo16, uint32_t lo8) {
     const u32x4 h = *(const u32x4*)q_at(tile, 4u * p, lo16);
-    const u32x2 l = *(const u32x2*)q_at(tile, 4u * P + 2u * p, lo8);
+    const u32x2 l = *(const u32x2*)q_at(tile, 4u * kQP + 2u * p, lo8);
     return i32x8{(int)h.x, (int)h.y, (int)h.z, (int)h.w, (int)l.x, (int)l.y, 0, 0};
 }
-template <uint32_t P>
 WL_DEV u32x2 q_scales(const uint8_t* tile, uint32_t lo8) {
-    return *(const u32x2*)q_at(tile, 6u * P, lo8);
+    return *(const u32x2*)q_at(tile, 6u * kQP, lo8);
 }
 // Two chunks of 64 columns of a row pair (lane (n, g): row 32 q + n + 16 (g >>
 // 1), block g & 1) -> 128 columns of each of its halves, in place.
@@ -408,16 +407,17 @@ WL_DEV void pair_swap(u32x4& x, u32x4& y) {
 // MB row blocks, KT k tiles per step: the slot holds tile (q, m), number MB q + m.
 // A DMA of a tile fills one of its kilobytes: 128 bytes of each of eight rows, a
 // row by eight lanes next to each other (lane l: row 8 h + l / 8). Wave v takes
-// kilobyte v of every tile; of a record of ten, the two left over of four tiles at
-// once: wave v kilobyte 8 + v % 2 of tile 4 x + v / 2 (past the tiles: out of
-// range, into the slot's end). (Lanes that took 64 bytes of each of 16 rows, every
+// kilobyte v of every tile, then one of the two left over of tile v / 2: kilobyte 8 +
+// v % 2 (past the tiles: out of range, into the slot's end). (Lanes that took 64 bytes of each of 16 rows, every
 // quarter wave 16 cache lines: 1000 tokens 1588 us a call, now 1556; 333 of hidden
 // 2944 309, 305; 7, 64 and 4096 the same within 0.4 %.) Absent rows, k tiles past the row's end and units past the record
 // land as zeros (zero scales too: their products are zero).
 template <uint32_t MB>
 struct AStreamQ {
     rsrc_t rs;
-    uint32_t base[MB], left, nk;  // lane byte offsets of the lane's rows (left: of its left-over groups' row), k tiles of a row
+    // lane byte offsets of the lane's units of its rows (left: of its left-over
+    // unit), k tiles of a row, bytes of a record
+    uint32_t base[MB], left, nk, rec;
 };
 // What the pipelines share: the layer's tables, the rows of a pass, the
 // epilogues. UP: gate/up of the routed experts, K = H, slices of 64 rows (tiles of
@@ -429,11 +429,10 @@ struct AStreamQ {
 template <bool UP, uint32_t NB, uint32_t KT>
 struct QBase {
     using AS = AStreamQ<NB>;
-    static constexpr uint32_t P = UP ? kQPUp : kQPDown, NG = (q6_units(P) + 3u) / 4u;  // groups of a record
-    static constexpr uint32_t kTiles = NB * KT, kTileB = 1024u * NG, kLeft = NG > 8u ? (kTiles + 3u) / 4u : 0u;
-    static constexpr uint32_t kDmas = kTiles + kLeft;
-    static_assert(NG == 8u || (NG == 10u && kLeft == 1u), "eight groups, or ten of at most four tiles");
-    static_assert(kTileB * kTiles + (kLeft ? 8192u : 0u) <= kSlotB, "a step's tiles fit a slot");
+    static constexpr uint32_t P = kQP, NG = (kQUnits + 3u) / 4u;  // groups of a record
+    static constexpr uint32_t kTiles = NB * KT, kTileB = 1024u * NG, kDmas = kTiles + 1u;
+    static_assert(NG == 10u && kTiles <= 4u, "ten groups of at most four tiles");
+    static_assert(kTileB * kTiles + 8192u <= kSlotB, "a step's tiles fit a slot");
     const DecodeArgs& a;
     const BatchArgs& b;
     uint32_t H, I, E, K, nk, S, nq, parts, nst, nst2, nu, v, lane, uoff;
@@ -444,6 +443,11 @@ struct QBase {
     const uint8_t* wbase;  // the weight stream's block and size (see SharedK)
     uint32_t wbytes, wpart, vw, vs, lo8, lo16;
     UnitInfo cu, un;     // the unit computed, the unit whose loads go out
+    // any row of the call has further pieces; the positions of these units among the
+    // work-group's, whether they run twice and are in their second run
+    bool any;
+    uint32_t ci, ni;
+    bool ctwice, csecond, ntwice, nsecond;
     const uint16_t *tt, *ent;  // UP: the token table; the entries where this kernel grouped them (or null)
 
     WL_MEM UnitInfo unit(uint32_t i) const {
@@ -459,46 +463,82 @@ struct QBase {
         x.row0 = ps.c0;
         return x;
     }
-    WL_MEM void bind(uint32_t i, AS& A) {
-        const UnitInfo x = un = unit(i);
+    // The activation row of row r (< nt) of unit i.
+    WL_MEM uint32_t row_of(const UnitInfo& x, uint32_t i, uint32_t r) const {
+        if (!UP) return x.row0 + r;
+        return x.e == a.E ? x.row0 + r - b.T * K : table_token(tt, b.tcap, kRB * NB, i, r, x.nt);
+    }
+    // A unit with a row of further pieces runs its steps twice: on the records, then
+    // on the further pieces.
+    WL_MEM bool twice(const UnitInfo& x, uint32_t i) const {
+        if (!any || !x.live) return false;
+        static_assert(kRB * NB <= 64u, "a lane per row");
+        const bool has = lane < x.nt && gld((UP ? b.more_up : b.more_dn) + row_of(x, i, min(lane, x.nt - 1u))) != 0u;
+        return __builtin_amdgcn_ballot_w64(has) != 0u;
+    }
+    // (called once for each run, in order)
+    WL_MEM void bind(uint32_t run, AS& A) {
+        nsecond = run > 0u && ntwice && !nsecond;
+        if (!nsecond) {
+            ni = run == 0u ? 0u : ni + 1u;
+            un = unit(ni);
+            ntwice = twice(un, ni);
+        }
+        const uint32_t i = ni;
+        const bool more = nsecond;
+        const UnitInfo x = un;
         const uint8_t* blk = x.live ? uni_ptr(stab[x.e]) : nullptr;
         wbase = blk;
         wbytes = blk ? (uint32_t)NL.total : 0u;
         wpart = x.part;
         const uint32_t kd = UP ? H : I, n = 8u * (v & 1u) + lane / 8u, c8 = lane % 8u ^ q_swizzle(n);
         const uint32_t nrow = UP ? b.T : b.T * (K + ((b.flags & kBatchShared4) ? 1u : 0u));
-        const uint32_t rowb = (uint32_t)q6_row_bytes(P, kd);
-        A.rs = make_rsrc(x.live ? (UP ? (const uint8_t*)b.norm : b.mid6) : nullptr, x.live ? nrow * rowb : 0u);
+        const uint32_t rec = (uint32_t)q6_row_bytes(kd), ext = (uint32_t)q6_more_bytes(kd);
+        const uint32_t rowb = UP ? rec + ext : more ? ext : rec, row0 = UP && more ? rec : 0u;
+        const uint8_t* rows = UP ? (const uint8_t*)b.norm : more ? b.mid6x : b.mid6;
+        A.rs = make_rsrc(x.live ? rows : nullptr, x.live ? nrow * rowb : 0u);
         A.nk = x.live ? nk : 0u;
-        auto row_at = [&](uint32_t m) {
+        A.rec = more ? kQMore : kQRecord;
+        // the lane's unit c of row m's record
+        auto row_at = [&](uint32_t m, uint32_t c) {
             const uint32_t r = kRB * m + n;
-            uint32_t row = x.row0 + r;
-            if (UP) row = x.e == a.E ? row - b.T * K : x.live ? table_token(tt, b.tcap, kRB * NB, i, r, x.nt) : 0u;
-            return r < x.nt ? row * rowb + 16u * c8 : kOOBV;
+            const uint32_t row = x.live ? row_of(x, i, r) : 0u;
+            bool has = r < x.nt && c < kQUnits;
+            if (more) {
+                has = has && gld((UP ? b.more_up : b.more_dn) + row) != 0u && q6_more_unit(c) != ~0u;
+                c = q6_more_unit(c);
+            }
+            return has ? row * rowb + row0 + 16u * c : kOOBV;
         };
 #pragma unroll
-        for (uint32_t m = 0; m < NB; m++) {
-            const uint32_t o = row_at(m);
-            A.base[m] = o == kOOBV ? o : o + 128u * (v / 2u);
-        }
-        if (kLeft) {
-            const uint32_t o = row_at(v / 2u % NB);
-            A.left = v / 2u < kTiles && 32u + c8 < q6_units(P) && o != kOOBV ? o + 512u : kOOBV;
-        }
+        for (uint32_t m = 0; m < NB; m++) A.base[m] = row_at(m, 8u * (v / 2u) + c8);
+        A.left = v / 2u < kTiles ? row_at(v / 2u % NB, 32u + c8) : kOOBV;
     }
     template <int SL>
     WL_MEM void dma(const AS& A, uint32_t s, uint32_t j) const {
         if (j < kTiles) {
             const uint32_t k = s * KT + j / NB;
-            dma16<SL>(A.rs, j * kTileB + v * 1024u, k < A.nk ? A.base[j % NB] : kOOBV, k * q6_record(P));
+            dma16<SL>(A.rs, j * kTileB + v * 1024u, k < A.nk ? A.base[j % NB] : kOOBV, k * A.rec);
         } else {
             const uint32_t t = v / 2u, k = s * KT + t / NB;
             dma16<SL>(A.rs, t < kTiles ? t * kTileB + (8u + v % 2u) * 1024u : kTiles * kTileB + v * 1024u,
-                      k < A.nk ? A.left : kOOBV, k * q6_record(P));
+                      k < A.nk ? A.left : kOOBV, k * A.rec);
         }
     }
-    WL_MEM void begin_unit(uint32_t i) {
-        cu = nst > 1u && i > 0u ? un : unit(i);  // (the loads are two steps ahead)
+    WL_MEM bool unit_end() {
+        csecond = ctwice && !csecond;
+        return !csecond;
+    }
+    WL_MEM void begin_unit(uint32_t run) {
+        ci = run == 0u ? 0u : ci + 1u;
+        csecond = false;
+        if (nst > 1u && run > 0u) {  // (the loads are two steps ahead)
+            cu = un;
+            ctwice = ntwice;
+        } else {
+            cu = unit(ci);
+            ctwice = twice(cu, ci);
+        }
         if (cu.live && stab[cu.e] == nullptr && threadIdx.x == 0) raise_error(a.sync, SyncMap::make(), E_NOT_RESIDENT, 0u);  // no waits in this path: epoch 0 aborts nothing
     }
     // The four slices of row block m, two at a time.
@@ -570,7 +610,7 @@ struct QNarrow : QBase<UP, NB, 2> {
         auto tile = [&](uint32_t q, uint32_t m) { return sl + (q * NB + m) * QB::kTileB; };
         auto frag = [&](uint32_t it) {
             const uint32_t m = it % NB, p = it / NB % P, q = it / (NB * P);
-            return q_frag<P>(tile(q, m), p, lo16, this->lo8);
+            return q_frag(tile(q, m), p, lo16, this->lo8);
         };
 #pragma unroll
         for (uint32_t it = 0; it < AH; it++) af[it] = frag(it);
@@ -579,7 +619,7 @@ struct QNarrow : QBase<UP, NB, 2> {
             const uint32_t m = it % NB, p = it / NB % P, q = it / (NB * P);
             if (p == 0u && m == 0u) {
 #pragma unroll
-                for (uint32_t i = 0; i < NB; i++) sa[i] = q_scales<P>(tile(q, i), this->lo8);
+                for (uint32_t i = 0; i < NB; i++) sa[i] = q_scales(tile(q, i), this->lo8);
                 if (!UP) {
 #pragma unroll
                     for (uint32_t h = 0; h < 2; h++) pair_swap(W.w[4u * q + h], W.w[4u * q + 2u + h]);
@@ -622,10 +662,9 @@ struct QNarrow : QBase<UP, NB, 2> {
     }
 };
 
-// Passes of three to five row blocks (down: four, six pieces take more LDS): bound
-// by the matrix cores and the loads' issue (750 to 900 cycles of MFMA per SIMD and
-// row block for a step's 32 KB of weights and 8 to 10 KB of rows per block). A
-// step is 128 columns.
+// Passes of three or four row blocks (a slot holds four tiles): bound by the matrix
+// cores and the loads' issue (900 cycles of MFMA per SIMD and row block for a step's
+// 32 KB of weights and 10 KB of rows per block). A step is 128 columns.
 template <bool UP, uint32_t NB>
 struct QWide : QBase<UP, NB, 1> {
     using QB = QBase<UP, NB, 1>;
@@ -664,11 +703,11 @@ struct QWide : QBase<UP, NB, 1> {
         i32x8 af[AH + 1u];
         u32x2 sa[NB];
         const uint32_t lo16 = this->lo16;
-        auto frag = [&](uint32_t it) { return q_frag<P>(sl + (it % NB) * QB::kTileB, it / NB, lo16, this->lo8); };
+        auto frag = [&](uint32_t it) { return q_frag(sl + (it % NB) * QB::kTileB, it / NB, lo16, this->lo8); };
 #pragma unroll
         for (uint32_t it = 0; it < AH; it++) af[it] = frag(it);
 #pragma unroll
-        for (uint32_t m = 0; m < NB; m++) sa[m] = q_scales<P>(sl + m * QB::kTileB, this->lo8);
+        for (uint32_t m = 0; m < NB; m++) sa[m] = q_scales(sl + m * QB::kTileB, this->lo8);
         // the step's scale bytes: UP the step's k tile of the word's two (byte 2
         // (i & 1)), down as the weights' halves (byte h)
         if (UP) {
@@ -794,9 +833,9 @@ WL_DEV ExpertTab load_expert_tab(const BatchArgs& b, uint32_t E, uint32_t K, uin
 // their units' count.
 template <bool UP, uint32_t NB>
 WL_DEV uint32_t run_routed(const DecodeArgs& a, const BatchArgs& b, uint32_t E, const ExpertTab& et,
-                           const uint8_t* const* stab, uint32_t uoff) {
+                           const uint8_t* const* stab, uint32_t uoff, bool any) {
     using Kn = std::conditional_t<(NB > 2u), QWide<UP, NB>, QNarrow<UP, NB>>;
-    const PassTab pt = load_pass_tab(et, E, UP ? kWideUp : kWideDown, NB);
+    const PassTab pt = load_pass_tab(et, E, NB);
     if (pt.n == 0u) return 0u;
     pipeline_drain();
     const uint32_t H = a.H, I = a.I;
@@ -813,6 +852,7 @@ WL_DEV uint32_t run_routed(const DecodeArgs& a, const BatchArgs& b, uint32_t E, 
     w.nst = NB > 2u ? w.nk : w.nst2;
     w.uoff = uoff % gridDim.x;
     const uint32_t U = pt.n * w.parts, b0 = (blockIdx.x + gridDim.x - w.uoff) % gridDim.x;
+    w.any = any;
     w.nu = U > b0 ? cdiv(U - b0, gridDim.x) : 0u;
     w.lane = threadIdx.x & 63u;
     w.v = uni(threadIdx.x >> 6);
@@ -836,8 +876,8 @@ WL_DEV uint32_t run_routed(const DecodeArgs& a, const BatchArgs& b, uint32_t E, 
 // Routed rows as fp6 pieces against fp4 weights run at 3.5 times the rate of bf16
 // pieces and need no conversion of the weights. Whole calls, hidden 6144, inter
 // 2048, 8 of 256 experts (256 work-groups of eight waves), before (bf16 pieces,
-// passes of 32 and 64) and now: 4096 tokens 8360 and 4900 us, 1000 tokens 2307 and
-// 1556, 64 tokens (one row block per expert; the weights' 4.4 GB at 6 TB/s) 751 and
+// passes of 32 and 64) and now: 4096 tokens 8360 and 5180 us, 1000 tokens 2307 and
+// 1601, 64 tokens (one row block per expert; the weights' 4.4 GB at 6 TB/s) 751 and
 // 757, 7 tokens 215.7 and 218.1; hidden 2944, inter 1408, 6 of 160 experts, 333 tokens: 462 and 305.
 // Error against 64 bits: 8.1e-7 and 4.5e-7 at 4096 tokens, 3.5e-7 and 1.5e-7 at 64.
 template <bool UP>
@@ -845,13 +885,13 @@ WL_DEV void run_gemm(const DecodeArgs* pa, const BatchArgs& b) {
     const DecodeArgs& a = *pa;
     uint8_t* dyn = dyn_lds();
     const bool sh4 = (b.flags & kBatchShared4) != 0u;
+    const bool any = uni(gld(b.more + (UP ? 0 : 1))) != 0u;
     const uint32_t E = a.E + (sh4 ? 1u : 0u);  // experts in the pass table
     const uint8_t* const* stab = load_slot_tab(a, a.E, sh4, (const uint8_t**)dyn);
     const ExpertTab et = load_expert_tab(b, E, a.K, (uint32_t*)(dyn + 8u * E), stab, UP);
     uint32_t u = run_shared_expert<UP>(a, b);
-    if constexpr (UP) u += run_routed<UP, 5>(a, b, E, et, stab, u);
-    u += run_routed<UP, 4>(a, b, E, et, stab, u);
-    u += run_routed<UP, 3>(a, b, E, et, stab, u);
-    u += run_routed<UP, 2>(a, b, E, et, stab, u);
-    run_routed<UP, 1>(a, b, E, et, stab, u);
+    u += run_routed<UP, 4>(a, b, E, et, stab, u, any);
+    u += run_routed<UP, 3>(a, b, E, et, stab, u, any);
+    u += run_routed<UP, 2>(a, b, E, et, stab, u, any);
+    run_routed<UP, 1>(a, b, E, et, stab, u, any);
 }

@@ -286,13 +286,16 @@ enum : uint32_t {
 };
 // launch_batched phases: routing (norm .. scatter), the GEMMs, the combine.
 enum : uint32_t { kPhaseRoute = 1u, kPhaseGemm = 2u, kPhaseCombine = 4u, kPhaseAll = 7u };
+// Bytes of 128 quantised columns (q6.h): a record and a record of further pieces.
+constexpr uint32_t kQRecord = 608, kQMore = 224;
 struct BatchArgs {
     uint32_t T;
     uint32_t flags;
     const float* hidden;   // [T][H] pre-norm residual stream
     const float* resid;    // [T][H] or null
     float* out;            // [T][H]
-    float* norm;           // [T][H]; after the top-k its quantised rows (q6.h: as many bytes)
+    float* norm;           // [T] rows of ldn floats: the f32 row; after the top-k the quantised one (q6.h)
+    uint32_t ldn;          // (its record and its further pieces)
     uint16_t* norm3;       // [T][3][H] bf16 pieces of norm
     float* logits;         // [T][E]
     int32_t* idx;          // [T][K]
@@ -303,6 +306,9 @@ struct BatchArgs {
     uint32_t* ent;         // [T*K] compact index -> token*K + slot (expert-major)
     uint32_t* pos;         // [T*K] token*K + slot -> compact index
     uint8_t* mid6;         // [T*K (+T)] quantised rows of midf (q6.h)
+    uint8_t* mid6x;        // their further pieces (in the space of norm3)
+    uint32_t *more_up, *more_dn;  // [T], [T*K (+T)]: the row has further pieces
+    uint32_t* more;        // [2]: any row of the gate/up inputs, of the SwiGLU values has
     uint32_t ldm;          // stride of the rows of midf and expout, which share their space row by row
     float* midf;           // [T*K (+T)][I] routed (and MXFP4 shared) SwiGLU outputs, compact rows
     float* expout;         // [T*K (+T)][H] routed (and MXFP4 shared) expert outputs, compact rows

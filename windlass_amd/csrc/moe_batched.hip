@@ -93,6 +93,7 @@ __global__ void __launch_bounds__(kThreads) bnorm_kernel(const DecodeArgs* __res
         hv[i] = __builtin_bit_cast(float4, bld16(hid_rs, 16u * j, 0u));
         lv[i] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(ln_rs, (int)(8u * j), 0, 0));
     }
+    if (t == 0u && tid < 2u) gst(b.more + tid, 0u);  // (the kernels after this one set them)
     const float rinv = norm_rinv(hv, red, H, a.eps);
 #pragma unroll
     for (int i = 0; i < kHV; i++) {
@@ -105,7 +106,7 @@ __global__ void __launch_bounds__(kThreads) bnorm_kernel(const DecodeArgs* __res
             o.y = norm_value(xs[1], rinv, a.ln_w != nullptr, ls[1]);
             o.z = norm_value(xs[2], rinv, a.ln_w != nullptr, ls[2]);
             o.w = norm_value(xs[3], rinv, a.ln_w != nullptr, ls[3]);
-            *(__attribute__((address_space(1))) u32x4*)(b.norm + (size_t)t * H + 4 * j) = __builtin_bit_cast(u32x4, o);
+            *(__attribute__((address_space(1))) u32x4*)(b.norm + (size_t)t * b.ldn + 4 * j) = __builtin_bit_cast(u32x4, o);
             const float os[4] = {o.x, o.y, o.z, o.w};
             if (!(b.flags & kBatchShared4)) store_pieces4(b.norm3 + (size_t)t * 3u * H + 4 * j, H, os);
         }
@@ -164,7 +165,7 @@ __global__ void __launch_bounds__(kThreads) broute_kernel(const DecodeArgs* __re
 #pragma unroll
     for (uint32_t tt = 0; tt < kTB; tt++) {
         const bool live = t0 + tt < b.T;
-        const rsrc_t nrs = make_rsrc(b.norm + (size_t)min(t0 + tt, b.T - 1u) * H, live ? H * 4u : 0u);
+        const rsrc_t nrs = make_rsrc(b.norm + (size_t)min(t0 + tt, b.T - 1u) * b.ldn, live ? H * 4u : 0u);
 #pragma unroll
         for (int m = 0; m < kRCH; m++) {
             const uint32_t c = tid + kThreads * m;
@@ -244,13 +245,15 @@ __global__ void __launch_bounds__(kThreads) broute_kernel(const DecodeArgs* __re
 }
 
 // The top-k of token t = blockIdx.x, and its normalised row, which the router
-// was the last to read, quantised in place (q6.h; same bytes as the f32 row).
+// was the last to read, quantised in place (q6.h).
 __global__ void __launch_bounds__(kThreads) btopk_kernel(const DecodeArgs* __restrict__ pa, const BatchArgs b) {
     const DecodeArgs& a = *pa;
     const uint32_t H = a.H, E = a.E, K = a.K, t = blockIdx.x, tid = threadIdx.x;
     __shared__ __align__(16) float row[(8192 / 32) * 36];  // 4 floats between blocks of 32: other banks
-    for (uint32_t j = tid; j < H / 4u; j += kThreads)
-        *(u32x4*)(row + 36u * (j / 8u) + 4u * (j % 8u)) = gld16(b.norm + (size_t)t * H + 4u * j);
+    __shared__ uint32_t more;
+    float* rowp = b.norm + (size_t)t * b.ldn;
+    for (uint32_t j = tid; j < H / 4u; j += kThreads) *(u32x4*)(row + 36u * (j / 8u) + 4u * (j % 8u)) = gld16(rowp + 4u * j);
+    if (tid == 0u) more = 0u;
     extern __shared__ __align__(16) uint8_t lds[];
     float* tk_sc = (float*)lds;
     float* tk_ch = tk_sc + E;
@@ -259,26 +262,34 @@ __global__ void __launch_bounds__(kThreads) btopk_kernel(const DecodeArgs* __res
     for (uint32_t e = tid; e < E; e += kThreads)
         topk_score(gld(b.logits + (size_t)t * E + e), gld(a.bias + e), e, tk_sc, tk_ch);
     lds_barrier();  // (every thread's reads of the row are done)
-    static_assert(q6_row_bytes(kQPUp, 128u) == 4u * 128u, "a quantised row takes its f32 row's place");
+    f32x16 even, odd;
     auto quantise = [&](uint32_t i) {
         if (i >= H / 32u) return;
-        f32x16 even, odd;
         q6_load(row + 36u * i, even, odd);
-        q6_store<kQPUp>((uint8_t*)(b.norm + (size_t)t * H) + (i / 4u) * q6_record(kQPUp), i % 4u, even, odd);
+        const uint32_t mx = q6_max(even, odd);
+        if (q6_wide(even, odd, mx)) more = 1u;
+        q6_store<false>((uint8_t*)rowp + (i / 4u) * kQRecord, i % 4u, even, odd, mx);
     };
     // up to 256 experts the argmax is wave 0's: the other waves quantise (at most
     // 256 blocks)
     if (E <= 256u) {
         if (tid < 64u) topk_argmax_wave(E, K, tk_sc, tk_ch, tk_idx, tk_w);
         else quantise(tid - 64u);
-        lds_barrier();
     } else {
         topk_rank(E, K, tk_sc, tk_ch, tk_idx, tk_w);
         quantise(tid);
     }
+    lds_barrier();
     if (tid < K) {
         gst(b.idx + (size_t)t * K + tid, (int32_t)tk_idx[tid]);
         gst(b.wts + (size_t)t * K + tid, topk_weight(a, K, tk_w, tid));
+    }
+    if (tid == 0u) gst(b.more_up + t, more);
+    if (more == 0u) return;
+    if (tid == 0u) gst(b.more, 1u);
+    if (tid < H / 32u) {
+        q6_load(row + 36u * tid, even, odd);
+        q6_store<true>((uint8_t*)rowp + q6_row_bytes(H) + (tid / 4u) * kQMore, tid % 4u, even, odd, q6_max(even, odd));
     }
 }
 
@@ -335,17 +346,17 @@ __global__ void __launch_bounds__(256) bscatter_kernel(const BatchArgs b, uint32
 
 // ---- pass table ----------------------------------------------------------------
 // An expert's tokens are cut into MFMA row blocks of 16, and those are split
-// evenly over passes of at most wb blocks (wb 5, 150 tokens: 10 blocks, 5 + 5).
+// evenly over passes of at most kWide blocks (100 tokens: 7 blocks, 4 + 3).
 constexpr uint32_t kRB = 16;                       // tokens of a row block
-constexpr uint32_t kWideUp = 5, kWideDown = 4;  // row blocks of the largest pass
+constexpr uint32_t kWide = 4;                      // row blocks of the largest pass
 struct PassSplit {
     uint32_t np, base, rem;  // passes; the first rem of them have base + 1 row blocks, the others base
     // the passes of nb row blocks and the first of them
     WL_MEM uint32_t count(uint32_t nb) const { return np == 0u ? 0u : base == nb ? np - rem : base + 1u == nb ? rem : 0u; }
     WL_MEM uint32_t first(uint32_t nb) const { return base == nb ? rem : 0u; }
 };
-WL_DEV PassSplit pass_split(uint32_t c, uint32_t wb) {
-    const uint32_t m = cdiv(c, kRB), np = cdiv(m, wb);
+WL_DEV PassSplit pass_split(uint32_t c) {
+    const uint32_t m = cdiv(c, kRB), np = cdiv(m, kWide);
     return np == 0u ? PassSplit{0u, 0u, 0u} : PassSplit{np, m / np, m % np};
 }
 // The experts' counts and offsets, in LDS, and room for the pass table.
@@ -361,16 +372,16 @@ struct ExpertTab {
 // to each other.
 struct PassTab {
     const uint32_t *cnt, *off, *pp;
-    uint32_t n, wb, nb;  // passes; row blocks of the largest pass and of these
+    uint32_t n, nb;  // passes; row blocks of each
 };
-WL_DEV PassTab load_pass_tab(const ExpertTab& et, uint32_t E, uint32_t wb, uint32_t nb) {
+WL_DEV PassTab load_pass_tab(const ExpertTab& et, uint32_t E, uint32_t nb) {
     const uint32_t tid = threadIdx.x;
     lds_barrier();  // the tables are written, the last pass table is no longer read
     if (tid < 64u) {
         const uint32_t per = cdiv(E, 64u), e0 = tid * per;
         uint32_t mine = 0;
         for (uint32_t i = 0; i < per; i++)
-            if (e0 + i < E) mine += pass_split(et.cnt[e0 + i], wb).count(nb);
+            if (e0 + i < E) mine += pass_split(et.cnt[e0 + i]).count(nb);
         uint32_t inc = mine;
 #pragma unroll
         for (uint32_t o = 1; o < 64u; o <<= 1) {
@@ -381,12 +392,12 @@ WL_DEV PassTab load_pass_tab(const ExpertTab& et, uint32_t E, uint32_t wb, uint3
         for (uint32_t i = 0; i < per; i++)
             if (e0 + i < E) {
                 et.pp[e0 + i] = run;
-                run += pass_split(et.cnt[e0 + i], wb).count(nb);
+                run += pass_split(et.cnt[e0 + i]).count(nb);
             }
         if (tid == 63u) et.pp[E] = inc;
     }
     lds_barrier();
-    return PassTab{et.cnt, et.off, et.pp, uni(et.pp[E]), wb, nb};
+    return PassTab{et.cnt, et.off, et.pp, uni(et.pp[E]), nb};
 }
 // Routed unit r (< n_passes * parts) -> (pass j, part). Units go in blocks
 // of 8 passes x parts, ordered so that unit r has j % 8 == r % 8 in full
@@ -419,7 +430,7 @@ WL_DEV uint32_t expert_of_pass(const uint32_t* pp, uint32_t E, uint32_t j) {
 }
 WL_DEV Pass pass_at(const PassTab& pt, uint32_t E, uint32_t j) {
     const uint32_t e = expert_of_pass(pt.pp, E, j), c = uni(pt.cnt[e]);
-    const PassSplit sp = pass_split(c, pt.wb);
+    const PassSplit sp = pass_split(c);
     const uint32_t p = sp.first(pt.nb) + j - uni(pt.pp[e]), r0 = kRB * (p * sp.base + min(p, sp.rem));
     return Pass{e, min(kRB * pt.nb, c - r0), uni(pt.off[e]) + r0};
 }
@@ -440,7 +451,7 @@ WL_DEV void fill_tokens(const Kn& k, uint16_t* tt, uint32_t W) {
     // wave v takes units v, v + kGW, ...: unit() takes a uniform index (it
     // reads the pass table through readfirstlane), lane m the pass rows m, m + 64
     const uint32_t v = uni(threadIdx.x >> 6), lane = threadIdx.x & 63u;
-    constexpr uint32_t R = 4, M = (kRB * kWideUp + 63u) / 64u;  // units per wave whose loads are in flight together
+    constexpr uint32_t R = 4, M = (kRB * kWide + 63u) / 64u;  // units per wave whose loads are in flight together
     for (uint32_t i0 = 0; i0 < k.nu; i0 += R * kGW) {
         uint32_t ent[R][M];
         bool has[R][M];
@@ -513,28 +524,43 @@ __global__ void __launch_bounds__(kGT) bdown_kernel(const DecodeArgs* __restrict
     run_gemm<false>(pa, b);
 }
 
-// The routed SwiGLU values (midf) as quantised rows (mid6): one block of 32
-// values per thread, staged through LDS so that the loads are coalesced.
-// 256 blocks per work-group.
+// The routed SwiGLU values (midf) as quantised rows (mid6, mid6x): a row per wave,
+// one block of 32 values per lane, staged through LDS so that the loads are
+// coalesced.
 __global__ void __launch_bounds__(256) bquant_kernel(const DecodeArgs* __restrict__ pa, const BatchArgs b) {
     const DecodeArgs& a = *pa;
-    const uint32_t I = a.I, nb = I / 32u, tid = threadIdx.x;
-    const uint32_t R = b.T * (a.K + ((b.flags & kBatchShared4) ? 1u : 0u)), N = R * nb;
-    __shared__ __align__(16) float xs[256 * 36];  // 32 values + 4: consecutive blocks in different banks
-    const uint32_t b0 = blockIdx.x * 256u;
-#pragma unroll
-    for (uint32_t i = 0; i < 8; i++) {
-        const uint32_t c = tid + 256u * i, blk = min(b0 + c / 8u, N - 1u);  // 16-byte chunk c % 8 of a block
-        *(u32x4*)(xs + 36u * (c / 8u) + 4u * (c % 8u)) =
-            gld16(b.midf + (size_t)(blk / nb) * b.ldm + 32u * (blk % nb) + 4u * (c % 8u));
-    }
-    lds_barrier();
-    const uint32_t blk = b0 + tid;
-    if (blk >= N) return;
+    const uint32_t I = a.I, nb = I / 32u, lane = threadIdx.x & 63u, v = uni(threadIdx.x >> 6);
+    const uint32_t R = b.T * (a.K + ((b.flags & kBatchShared4) ? 1u : 0u)), row = blockIdx.x * 4u + v;
+    __shared__ __align__(16) float xs[4][64 * 36];  // 32 values + 4: consecutive blocks in different banks
+    const float* mid = b.midf + (size_t)min(row, R - 1u) * b.ldm;
     f32x16 even, odd;
-    q6_load(xs + 36u * tid, even, odd);
-    const uint32_t row = blk / nb, kb = blk % nb;
-    q6_store<kQPDown>(b.mid6 + (size_t)row * q6_row_bytes(kQPDown, I) + (kb / 4u) * q6_record(kQPDown), kb % 4u, even, odd);
+    bool wide = false;
+    for (uint32_t b0 = 0; b0 < nb; b0 += 64u) {
+#pragma unroll
+        for (uint32_t i = 0; i < 8; i++) {
+            const uint32_t c = lane + 64u * i;  // 16-byte chunk c % 8 of block c / 8
+            *(u32x4*)(xs[v] + 36u * (c / 8u) + 4u * (c % 8u)) = gld16(mid + 32u * min(b0 + c / 8u, nb - 1u) + 4u * (c % 8u));
+        }
+        lds_barrier();
+        const uint32_t k = b0 + lane;
+        if (row < R && k < nb) {
+            q6_load(xs[v] + 36u * lane, even, odd);
+            const uint32_t mx = q6_max(even, odd);
+            wide |= q6_wide(even, odd, mx);
+            q6_store<false>(b.mid6 + (size_t)row * q6_row_bytes(I) + (k / 4u) * kQRecord, k % 4u, even, odd, mx);
+        }
+        lds_barrier();
+    }
+    const bool more = __builtin_amdgcn_ballot_w64(wide) != 0u;
+    if (row < R && lane == 0u) {
+        gst(b.more_dn + row, more ? 1u : 0u);
+        if (more) gst(b.more + 1, 1u);
+    }
+    if (row >= R || !more) return;
+    for (uint32_t k = lane; k < nb; k += 64u) {
+        q6_load(mid + 32u * k, even, odd);
+        q6_store<true>(b.mid6x + (size_t)row * q6_more_bytes(I) + (k / 4u) * kQMore, k % 4u, even, odd, q6_max(even, odd));
+    }
 }
 
 // out[t] = (resid[t] +) sum_k w[t][k] e_k[t] in slot order + shared[t]
@@ -580,7 +606,7 @@ static uint32_t batched_tok_entries(uint32_t T, uint32_t I, uint32_t E, uint32_t
     auto cd = [](uint64_t a, uint64_t b) { return (a + b - 1u) / b; };
     const uint64_t R = (uint64_t)T * (K + 1u), NS = cd(I / kSlice, 4u);
     uint64_t most = 0;
-    for (uint32_t nb = 1; nb <= kWideUp; nb++) {
+    for (uint32_t nb = 1; nb <= kWide; nb++) {
         uint64_t n = R / (kRB * (nb - 1u) + 1u);
         if (nb <= 2u) n = std::min<uint64_t>(n, E + 1u);
         most = std::max(most, cd(n * NS, grid) * kRB * nb);
@@ -655,7 +681,7 @@ int launch_batched(const DecodeArgs* d_args, const BatchArgs& b, uint32_t H, uin
         const uint32_t gu = resident(up, up_lds), gd = resident(down, gemm_lds);
         const uint32_t rows = b.T * (K + ((b.flags & kBatchShared4) ? 1u : 0u));
         hipLaunchKernelGGL(bup_kernel, dim3(gu), dim3(kGT), up_lds, s, d_args, bt);
-        hipLaunchKernelGGL(bquant_kernel, dim3((uint32_t)(((uint64_t)rows * (I / 32u) + 255u) / 256u)), dim3(256), 0, s, d_args, bt);
+        hipLaunchKernelGGL(bquant_kernel, dim3((rows + 3u) / 4u), dim3(256), 0, s, d_args, bt);
         hipLaunchKernelGGL(bdown_kernel, dim3(gd), dim3(kGT), gemm_lds, s, d_args, bt);
     }
     if (phases & kPhaseCombine)

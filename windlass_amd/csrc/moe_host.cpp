@@ -1128,8 +1128,17 @@ static size_t batch_layout(const wl_ctx* c, uint32_t T, uint8_t* base, wl::Batch
     };
     wl::BatchArgs d{};
     wl::BatchArgs& x = b ? *b : d;
-    take(&x.norm, 4 * t * H);
-    take(&x.norm3, 6 * t * H);
+    const size_t Kr = K + (c->any_sh4 ? 1u : 0u);  // + the MXFP4 shared expert's rows
+    const size_t ldn = (wl::kQRecord + wl::kQMore) * (H / 128u);
+    x.ldn = (uint32_t)(ldn / 4u);
+    take(&x.norm, t * ldn);
+    // (the bf16 shared expert's gate/up is the last to read norm3, before any
+    // SwiGLU value is quantised)
+    take(&x.norm3, t * std::max(6 * H, wl::kQMore * Kr * (I / 128u)));
+    x.mid6x = (uint8_t*)x.norm3;
+    take(&x.more, 8);
+    take(&x.more_up, 4 * t);
+    take(&x.more_dn, 4 * t * Kr);
     take(&x.logits, 4 * t * E);
     take(&x.idx, 4 * t * K);
     take(&x.wts, 4 * t * K);
@@ -1138,8 +1147,9 @@ static size_t batch_layout(const wl_ctx* c, uint32_t T, uint8_t* base, wl::Batch
     take(&x.lists, 4 * E * t);
     take(&x.ent, 4 * t * K);
     take(&x.pos, 4 * t * K);
-    const size_t Kr = K + (c->any_sh4 ? 1u : 0u);  // + the MXFP4 shared expert's rows
-    take(&x.mid6, 6 * t * Kr * I);  // (records of 4.75 bytes per value; this size keeps the chunks of the static scratch)
+    // (more than its records where that keeps the chunks of the static scratch at
+    // what they were with 6 bytes a value here and 4 in norm)
+    take(&x.mid6, t * std::max(wl::kQRecord * Kr * (I / 128u), 6 * Kr * I - std::min(6 * Kr * I, ldn - 4 * H)));
     // a row's SwiGLU values are read before its output is written (and no
     // other row's output lies there): they share its space
     x.ldm = (uint32_t)std::max(I, H);

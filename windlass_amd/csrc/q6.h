@@ -1,35 +1,49 @@
-// q6.h — f32 rows in five 6-bit floating-point pieces, the operands of the
+// q6.h — f32 rows in six 6-bit floating-point pieces, the operands of the
 // routed experts' GEMMs on gfx950's scaled matrix instruction (batched_gemm.h).
 //
 // v_mfma_scale_f32_16x16x128_f8f6f4 takes the MXFP4 weights as they lie in the
 // native block (a lane's 16 bytes are its 32 values, its E8M0 byte the scale
-// operand), so nothing is converted. The f32 activations run as P 6-bit
+// operand), so nothing is converted. The f32 activations run as 6-bit
 // floating-point pieces (E2M3) per block of 32 values, x = sum of p_i 2^s_i:
 // s_1 puts the block's largest value in (3.75, 7.5], each piece takes the
 // nearest E2M3 value of what the pieces before it left, and the scales fall by
 // 4, then 5 powers of two a piece, which is what a piece's rounding leaves (at
-// most 1/4 after the first, 1/8 of its scale after the others). Five pieces
-// leave at most 2^-24 of the block's largest value, an f32 rounding of it:
-// enough for the normalised input of gate/up. The SwiGLU values within a block
-// differ by more; six pieces (2^-29) keep full f32 precision down to 1/32 of
-// the block's largest value, and down projections whose weights single out a
-// small value stay within 1e-5 of it (tests/test_gpu_e8m0_corners.py).
+// most 1/4 after the first, 1/8 of its scale after the others). Six pieces leave
+// at most 2^-29 of the block's largest value: full f32 precision down to 1/32 of
+// it, 21 bits down to 1/256.
 //
-// Why: measured on MI355X the instruction runs 8.5 PFLOP/s with 6-bit against
-// 4-bit operands (bf16 2.43, 8-bit 4.8), so five or six pieces cost 0.5 to 0.6
-// of the three bf16 pieces' matrix time, and with 4- and 6-bit operands its sums
-// keep f32 precision (a probe: exact while the terms span 2^21, as the f32
-// accumulator). The GEMMs that ran three bf16 pieces against weights converted
-// to bf16 were bound by those MFMAs, the conversions and the LDS reads (12 KB
-// per 16 tokens and 128 columns, 7.5 and 9 KB here).
+// That is enough for a block whose values are of one size. Where most lie far below
+// a few (q6_wide), as beside the outlier channels of a trained model, weights that
+// are zero at those few (MXFP4 rounds many to zero) leave a sum of the small ones
+// alone; with five pieces such sums were off by 3e-6 of the largest output at 100
+// times, 1e-3 at 30000 times, and six leave a 32nd of that. A row with such a block
+// therefore has two further pieces per block, in records of their own that the GEMMs
+// run as a second pass over the same weights, into the same sums: 2^-39 of the
+// largest value, full f32 precision down to 1/32768 of it. The test counts values
+// rather than looking at the smallest: SwiGLU values are products, and some of any
+// 32 are small. Normal inputs and the SwiGLU values they make take none (4096 tokens
+// of hidden 6144). Units with such rows run twice as long (hidden 6144, inter 2048, 8
+// of 256 experts, 12 columns 1000 times the rest in one token, or in every one: 7
+// tokens 247 and 306 us, without 214; 1000 tokens 1646 and 2290, 1601; 4096 tokens
+// 5263 and 7135, 5180).
+//
+// Why this format: measured on MI355X the instruction runs 8.5 PFLOP/s with 6-bit
+// against 4-bit operands (bf16 2.43, 8-bit 4.8), so six pieces cost 0.6 of three
+// bf16 pieces' matrix time, and with 4- and 6-bit operands its sums keep f32
+// precision (a probe: exact while the terms span 2^21, as the f32 accumulator). The
+// GEMMs that ran three bf16 pieces against weights converted to bf16 were bound by
+// those MFMAs, the conversions and the LDS reads (12 KB per 16 tokens and 128
+// columns, 9 KB here). The sixth piece of the gate/up inputs takes 1 % at 256
+// tokens, 4 % at 1000 and 7 % at 4096 (1533 to 1601 and 4836 to 5180 us).
 //
 // A quantised row is a record per 128 columns (k tile) of 16-byte units c: c =
 // 4p + g the first 16 bytes of piece p of block g, c = 4P + 2p + h the last 8
 // bytes of piece p of blocks 2h and 2h + 1, c = 6P + h the scale bytes (8 per
-// block, P used) of blocks 2h and 2h + 1: 512 bytes for five pieces, 608 for
-// six. A DMA into LDS takes eight units of each of eight rows.
+// block, P used) of blocks 2h and 2h + 1: 608 bytes for P = 6, 224 for P = 2. A DMA
+// into LDS takes eight units of each of eight rows.
 #pragma once
 #include "dev_common.h"
+#include "internal.h"
 
 namespace wl {
 
@@ -39,40 +53,70 @@ typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(32))) float f32x32;
 
-constexpr uint32_t kQPUp = 5, kQPDown = 6;  // pieces of the gate/up inputs and of the SwiGLU values
-__host__ __device__ constexpr uint32_t q6_units(uint32_t P) { return 6u * P + 2u; }
-__host__ __device__ constexpr uint32_t q6_record(uint32_t P) { return 16u * q6_units(P); }
+constexpr uint32_t kQP = 6, kQX = 2;  // pieces of a record, further pieces
+constexpr uint32_t kQUnits = 6u * kQP + 2u;
+static_assert(16u * kQUnits == kQRecord && 16u * (6u * kQX + 2u) == kQMore, "record sizes");
 // bytes of a row of k columns
-__host__ __device__ constexpr size_t q6_row_bytes(uint32_t P, uint32_t k) { return (size_t)q6_record(P) * (k / 128u); }
+__host__ __device__ constexpr size_t q6_row_bytes(uint32_t k) { return (size_t)kQRecord * (k / 128u); }
+__host__ __device__ constexpr size_t q6_more_bytes(uint32_t k) { return (size_t)kQMore * (k / 128u); }
+// Where unit c of a record lies in the record of further pieces, whose pieces are
+// read as the first of a record that has no others (or ~0: a zero unit).
+__host__ __device__ constexpr uint32_t q6_more_unit(uint32_t c) {
+    return c < 4u * kQX                                 ? c
+           : c >= 4u * kQP && c < 4u * kQP + 2u * kQX ? c - 4u * kQP + 4u * kQX
+           : c >= 6u * kQP && c < 6u * kQP + 2u       ? c - 6u * kQP + 6u * kQX
+                                                      : ~0u;
+}
 
-// Block g of a k tile: 32 values (even[i], odd[i] columns 2i and 2i + 1) into
-// its parts of the record at rec.
-template <uint32_t P>
-WL_DEV void q6_store(uint8_t* rec, uint32_t g, f32x16 even, f32x16 odd) {
+// The largest magnitude of a block, as bits.
+WL_DEV uint32_t q6_max(const f32x16& even, const f32x16& odd) {
     uint32_t mx = 0u;
 #pragma unroll
     for (int i = 0; i < 16; i++) {
         mx = max(mx, __float_as_uint(even[i]) & 0x7FFFFFFFu);
         mx = max(mx, __float_as_uint(odd[i]) & 0x7FFFFFFFu);
     }
+    return mx;
+}
+// Whether a block of largest magnitude mx takes further pieces: at most eight of
+// its values are within 2^8 of the largest and smaller ones are there, or twelve lie
+// under 2^-12 of it.
+WL_DEV bool q6_wide(const f32x16& even, const f32x16& odd, uint32_t mx) {
+    const float m = __uint_as_float(mx), lim = m * 0x1p-8f, lim2 = m * 0x1p-12f;
+    uint32_t large = 0u, zero = 0u, tiny = 0u;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const float a = fabsf(even[i]), b = fabsf(odd[i]);
+        large += (a >= lim ? 1u : 0u) + (b >= lim ? 1u : 0u);
+        zero += (a == 0.f ? 1u : 0u) + (b == 0.f ? 1u : 0u);
+        tiny += (a < lim2 ? 1u : 0u) + (b < lim2 ? 1u : 0u);
+    }
+    return mx < 0x7F800000u && ((large <= 8u && large + zero < 32u) || tiny >= zero + 12u);
+}
+// Block g of a k tile: 32 values (even[i], odd[i] columns 2i and 2i + 1) of largest
+// magnitude mx into its parts of the record at rec, or (MORE) its further pieces
+// into theirs.
+template <bool MORE>
+WL_DEV void q6_store(uint8_t* rec, uint32_t g, f32x16 even, f32x16 odd, uint32_t mx) {
     // biased exponent of s_1: the largest value over it is in (3.75, 7.5]; large
-    // enough that all scales are normal powers of two (a block of values under
-    // 2^-100 keeps what that leaves of it)
-    constexpr uint32_t drop[6] = {0u, 4u, 9u, 14u, 19u, 24u}, lo = drop[P - 1u] + 1u;
+    // enough that all scales of a record are normal powers of two (a block of values
+    // under 2^-100 keeps what that leaves of it: to 2^-129)
+    constexpr uint32_t kFirst = MORE ? kQP : 0u, kEnd = MORE ? kQP + kQX : kQP, PN = kEnd - kFirst;
+    constexpr uint32_t lo = 5u * (kQP - 1u);
     uint32_t e = (mx >> 23) + ((mx & 0x7FFFFFu) > 0x700000u ? 1u : 0u);
     e = e < lo + 2u ? lo : e - 2u;
     const bool bad = mx >= 0x7F800000u;  // an infinity or a NaN: the E8M0 NaN, and NaN sums
     uint64_t sc = 0;
 #pragma unroll
-    for (uint32_t p = 0; p < P; p++) {
-        const uint32_t ep = e - drop[p];
+    for (uint32_t p = 0; p < kEnd; p++) {
+        const uint32_t drop = p ? 5u * p - 1u : 0u, ep = e > drop ? e - drop : 1u;
         const float s = __uint_as_float(ep << 23);
         // Both conversions take several passes and must not write over what they
         // still have to read (a fifth piece whose result the compiler had put
         // over its scale came out wrong), so their operands stay live.
         const u32x6 q = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(even, odd, s);
         asm volatile("" ::"v"(q), "v"(even), "v"(odd), "v"(s));
-        if (p + 1u < P) {
+        if (p + 1u < kEnd) {
             const f32x32 y = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(q, s);
             asm volatile("" ::"v"(y), "v"(q), "v"(s));
 #pragma unroll
@@ -81,11 +125,13 @@ WL_DEV void q6_store(uint8_t* rec, uint32_t g, f32x16 even, f32x16 odd) {
                 odd[i] -= y[2 * i + 1];
             }
         }
-        sc |= (uint64_t)(bad ? 255u : ep) << (8u * p);
-        gst((u32x4*)(rec + 16u * (4u * p + g)), u32x4{q[0], q[1], q[2], q[3]});
-        gst((uint64_t*)(rec + 16u * (4u * P + 2u * p + (g >> 1)) + 8u * (g & 1u)), (uint64_t)q[4] | ((uint64_t)q[5] << 32));
+        if (p < kFirst) continue;
+        const uint32_t pi = p - kFirst;
+        sc |= (uint64_t)(bad ? 255u : ep) << (8u * pi);
+        gst((u32x4*)(rec + 16u * (4u * pi + g)), u32x4{q[0], q[1], q[2], q[3]});
+        gst((uint64_t*)(rec + 16u * (4u * PN + 2u * pi + (g >> 1)) + 8u * (g & 1u)), (uint64_t)q[4] | ((uint64_t)q[5] << 32));
     }
-    gst((uint64_t*)(rec + 16u * (6u * P + (g >> 1)) + 8u * (g & 1u)), sc);
+    gst((uint64_t*)(rec + 16u * (6u * PN + (g >> 1)) + 8u * (g & 1u)), sc);
 }
 // The 32 values at x (16-byte aligned), split into even and odd columns.
 WL_DEV void q6_load(const float* x, f32x16& even, f32x16& odd) {
