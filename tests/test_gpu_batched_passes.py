@@ -43,3 +43,21 @@ def test_passes_at_block_edges(gpu, T, shape):
         if t in (0, T - 1):
             assert O.rel_to_scale(O.moe_layer(hs[t], dm.dense[0], src, 0, c)["out"], out[t]) < TOL, t
     dm.close()
+
+
+@pytest.mark.parametrize("E,K,T", [(48, 1, 512), (48, 1, 513), (624, 1, 512), (640, 1, 512), (48, 8, 64), (16, 16, 32),
+                                   (624, 2, 31)])
+def test_entries_grouped_by_expert(gpu, E, K, T):
+    """Up to 512 entries are grouped inside the gate/up kernel (a bit per token and
+    expert; up to 624 experts), more of them, or more experts, by kernels of their
+    own. Hidden 256 and inter 128: a unit is one step. Counts equal the ids'; every
+    seventh token and the last agree with the decode path."""
+    c = dict(SMALL, hidden=256, moe_inter=128, n_routed_experts=E, n_experts_per_tok=K)
+    dm = DeviceModel(c, seed=22, n_layers=1)
+    hs = _tokens(256, T, 2200 + T)
+    out = _batched(dm, hs)
+    _, ids, _ = dm.ctx.batched_routing(T)
+    assert np.array_equal(dm.ctx.batched_counts(), np.bincount(ids.reshape(-1), minlength=E))
+    for t in [*range(0, T, 7), T - 1]:
+        assert O.rel_to_scale(_decode(dm, hs[t]), out[t]) < TOL, t
+    dm.close()

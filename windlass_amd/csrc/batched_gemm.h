@@ -448,7 +448,7 @@ struct QBase {
     bool any;
     uint32_t ci, ni;
     bool ctwice, csecond, ntwice, nsecond;
-    const uint16_t *tt, *ent;  // UP: the token table; the entries where this kernel grouped them (or null)
+    const uint16_t* tt;  // UP: the token table, or the tokens of all entries where this kernel grouped them
 
     WL_MEM UnitInfo unit(uint32_t i) const {
         UnitInfo x{false, 0u, 0u, 0u, 0u};
@@ -466,7 +466,8 @@ struct QBase {
     // The activation row of row r (< nt) of unit i.
     WL_MEM uint32_t row_of(const UnitInfo& x, uint32_t i, uint32_t r) const {
         if (!UP) return x.row0 + r;
-        return x.e == a.E ? x.row0 + r - b.T * K : table_token(tt, b.tcap, kRB * NB, i, r, x.nt);
+        if (x.e == a.E) return x.row0 + r - b.T * K;
+        return b.group ? (uint32_t)tt[x.row0 + min(r, x.nt - 1u)] : table_token(tt, b.tcap, kRB * NB, i, r, x.nt);
     }
     // A unit with a row of further pieces runs its steps twice: on the records, then
     // on the further pieces.
@@ -751,29 +752,42 @@ struct QWide : QBase<UP, NB, 1> {
 
 // Calls of at most kGroupMax entries that run all phases (BatchArgs::group): the
 // work-groups of bup_kernel find the experts' counts, offsets and entries from the
-// ids by themselves, one entry per thread (its rank: the entries of its expert
-// before it), and the first also stores them for the kernels after it. bcount and
-// bscatter, a launch of 5 us each, take all other calls.
-constexpr uint32_t kGroupMax = kGT;
-// The LDS of the grouped entries, after the token table.
-__host__ __device__ inline size_t ent_table_offset(uint32_t E, uint32_t tcap) { return tok_table_offset(E) + 2u * (size_t)tcap; }
+// ids by themselves, and the first also stores them for the kernels after it. bcount
+// and bscatter, a launch of 5 us each, take all other calls. An expert is chosen at
+// most once per token, so a bit per token and expert gives counts and ranks
+// (comparing every entry with all before it took 9 us at 64 tokens of 8 experts, all
+// of it before the first load of a weight).
+constexpr uint32_t kGroupMax = 4u * kGT;
+// Words of token bits of an expert; they have to fit a slot.
+__host__ __device__ inline uint32_t group_words(uint32_t T) { return (T + 31u) / 32u; }
+// Afterwards ent[r] is the token of compact entry r (in the place of the token table).
 WL_DEV void group_entries(const BatchArgs& b, uint32_t E, uint32_t K, const ExpertTab& et, uint16_t* ent) {
-    const uint32_t n = b.T * K, i = threadIdx.x, lane = i & 63u;
-    uint32_t* ids = (uint32_t*)slot<0>();  // (free until the first pipeline)
-    const uint32_t id = i < n ? (uint32_t)gld(b.idx + i) : ~0u;
-    ids[i] = id;
-    for (uint32_t f = i; f < E; f += kGT) et.cnt[f] = 0u;
+    constexpr uint32_t N = kGroupMax / kGT;
+    const uint32_t n = b.T * K, i = threadIdx.x, lane = i & 63u, nw = group_words(b.T);
+    uint32_t* bits = (uint32_t*)slot<0>();  // (free until the first pipeline)
+    uint32_t id[N], t[N], rank[N];
+#pragma unroll
+    for (uint32_t r = 0; r < N; r++) {
+        t[r] = (i + r * kGT) / K;
+        id[r] = i + r * kGT < n ? (uint32_t)gld(b.idx + i + r * kGT) : 0u;
+    }
+    for (uint32_t f = i; f < E * nw; f += kGT) bits[f] = 0u;
     lds_barrier();
-    if (i < n) atomicAdd(et.cnt + id, 1u);
-    uint32_t rank = 0;
-    const uint32_t nb = min(n, uni(i | 63u) + 1u);  // (entries past n are no expert's)
-#pragma unroll 1
-    for (uint32_t j = 0; j < nb; j += 32u) {
-        u32x4 q[8];
 #pragma unroll
-        for (uint32_t r = 0; r < 8; r++) q[r] = *(const u32x4*)(ids + j + 4u * r);
+    for (uint32_t r = 0; r < N; r++)
+        if (i + r * kGT < n) atomicOr(bits + id[r] * nw + t[r] / 32u, 1u << (t[r] % 32u));
+    lds_barrier();
+    for (uint32_t f = i; f < E; f += kGT) {
+        uint32_t c = 0;
+        for (uint32_t w = 0; w < nw; w++) c += (uint32_t)__popc(bits[f * nw + w]);
+        et.cnt[f] = c;
+    }
 #pragma unroll
-        for (uint32_t r = 0; r < 32; r++) rank += q[r / 4u][r % 4u] == id && j + r < i ? 1u : 0u;
+    for (uint32_t r = 0; r < N; r++) {
+        rank[r] = 0u;
+        if (i + r * kGT >= n) continue;
+        for (uint32_t w = 0; w < t[r] / 32u; w++) rank[r] += (uint32_t)__popc(bits[id[r] * nw + w]);
+        rank[r] += (uint32_t)__popc(bits[id[r] * nw + t[r] / 32u] & ((1u << (t[r] % 32u)) - 1u));
     }
     lds_barrier();
     if (i < 64u) {
@@ -783,8 +797,8 @@ WL_DEV void group_entries(const BatchArgs& b, uint32_t E, uint32_t K, const Expe
         uint32_t inc = mine;
 #pragma unroll
         for (uint32_t o = 1; o < 64u; o <<= 1) {
-            const uint32_t t = __shfl_up(inc, o, 64);
-            if (lane >= o) inc += t;
+            const uint32_t t0 = __shfl_up(inc, o, 64);
+            if (lane >= o) inc += t0;
         }
         uint32_t off = inc - mine;
         for (uint32_t f = e0; f < min(e0 + per, E); f++) {
@@ -794,12 +808,15 @@ WL_DEV void group_entries(const BatchArgs& b, uint32_t E, uint32_t K, const Expe
     }
     lds_barrier();
     const bool put = blockIdx.x == 0u;
-    if (i < n) {
-        const uint32_t r = et.off[id] + rank;
-        ent[r] = (uint16_t)i;
+#pragma unroll
+    for (uint32_t r = 0; r < N; r++) {
+        const uint32_t en = i + r * kGT;
+        if (en >= n) continue;
+        const uint32_t c = et.off[id[r]] + rank[r];
+        ent[c] = (uint16_t)t[r];
         if (put) {
-            gst(b.ent + r, i);
-            gst(b.pos + i, r);
+            gst(b.ent + c, en);
+            gst(b.pos + en, c);
         }
     }
     if (!put) return;
@@ -811,22 +828,30 @@ WL_DEV void group_entries(const BatchArgs& b, uint32_t E, uint32_t K, const Expe
 }
 WL_DEV ExpertTab load_expert_tab(const BatchArgs& b, uint32_t E, uint32_t K, uint32_t* s, const uint8_t* const* stab,
                                  bool up) {
-    const ExpertTab et{s, s + E, s + 2u * E};
+    const ExpertTab et{s, s + E, s + 2u * E, s + 3u * E + 1u};
     const bool skip = (b.flags & kBatchSkipUnbound) != 0u;
     const uint32_t esh = (b.flags & kBatchShared4) ? E - 1u : E;
     const bool group = up && b.group != 0u;
-    if (group) group_entries(b, esh, K, et, (uint16_t*)(dyn_lds() + ent_table_offset(esh, b.tcap)));
+    if (group) group_entries(b, esh, K, et, (uint16_t*)(dyn_lds() + tok_table_offset(esh)));
+    uint32_t sizes = 0;
     for (uint32_t f = threadIdx.x; f < E; f += kGT) {
+        uint32_t c;
         if (f == esh) {
-            et.cnt[f] = (b.flags & kBatchNoShared) ? 0u : b.T;
+            c = (b.flags & kBatchNoShared) ? 0u : b.T;
             et.off[f] = b.T * K;
-            continue;
+        } else if (group) {
+            c = et.cnt[f];
+        } else {
+            // stab[f] was written by this thread (load_slot_tab, same stride)
+            c = skip && stab[f] == nullptr ? 0u : gld(b.counts + f);
+            et.off[f] = gld(b.offsets + f);
         }
-        if (group) continue;
-        // stab[f] was written by this thread (load_slot_tab, same stride)
-        et.cnt[f] = skip && stab[f] == nullptr ? 0u : gld(b.counts + f);
-        et.off[f] = gld(b.offsets + f);
+        et.cnt[f] = c;
+        sizes |= pass_split(c).sizes();
     }
+#pragma unroll
+    for (uint32_t o = 1; o < 64u; o <<= 1) sizes |= __shfl_xor(sizes, (int)o, 64);
+    if ((threadIdx.x & 63u) == 0u) et.sizes[threadIdx.x >> 6] = sizes;
     return et;
 }
 // The routed passes of NB row blocks, starting at work-group uoff; returns
@@ -836,7 +861,6 @@ WL_DEV uint32_t run_routed(const DecodeArgs& a, const BatchArgs& b, uint32_t E, 
                            const uint8_t* const* stab, uint32_t uoff, bool any) {
     using Kn = std::conditional_t<(NB > 2u), QWide<UP, NB>, QNarrow<UP, NB>>;
     const PassTab pt = load_pass_tab(et, E, NB);
-    if (pt.n == 0u) return 0u;
     pipeline_drain();
     const uint32_t H = a.H, I = a.I;
     Kn w(a, b);
@@ -866,8 +890,7 @@ WL_DEV uint32_t run_routed(const DecodeArgs& a, const BatchArgs& b, uint32_t E, 
     if (UP) {
         uint16_t* tt = (uint16_t*)(dyn_lds() + tok_table_offset(a.E));
         w.tt = tt;
-        w.ent = b.group ? (const uint16_t*)(dyn_lds() + ent_table_offset(a.E, b.tcap)) : nullptr;
-        fill_tokens(w, tt, kRB * NB);
+        if (!b.group) fill_tokens(w, tt, kRB * NB);
     }
     run_units(w);
     return U;
@@ -890,8 +913,15 @@ WL_DEV void run_gemm(const DecodeArgs* pa, const BatchArgs& b) {
     const uint8_t* const* stab = load_slot_tab(a, a.E, sh4, (const uint8_t**)dyn);
     const ExpertTab et = load_expert_tab(b, E, a.K, (uint32_t*)(dyn + 8u * E), stab, UP);
     uint32_t u = run_shared_expert<UP>(a, b);
-    u += run_routed<UP, 4>(a, b, E, et, stab, u, any);
-    u += run_routed<UP, 3>(a, b, E, et, stab, u, any);
-    u += run_routed<UP, 2>(a, b, E, et, stab, u, any);
-    run_routed<UP, 1>(a, b, E, et, stab, u, any);
+    // (pass sizes that no expert has cost a table of 2 us each where they were
+    // looked up one by one)
+    lds_barrier();
+    uint32_t sizes = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kGW; w++) sizes |= et.sizes[w];
+    sizes = uni(sizes);
+    if (sizes & 1u << 4) u += run_routed<UP, 4>(a, b, E, et, stab, u, any);
+    if (sizes & 1u << 3) u += run_routed<UP, 3>(a, b, E, et, stab, u, any);
+    if (sizes & 1u << 2) u += run_routed<UP, 2>(a, b, E, et, stab, u, any);
+    if (sizes & 1u << 1) run_routed<UP, 1>(a, b, E, et, stab, u, any);
 }

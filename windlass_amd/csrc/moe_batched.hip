@@ -354,6 +354,8 @@ struct PassSplit {
     // the passes of nb row blocks and the first of them
     WL_MEM uint32_t count(uint32_t nb) const { return np == 0u ? 0u : base == nb ? np - rem : base + 1u == nb ? rem : 0u; }
     WL_MEM uint32_t first(uint32_t nb) const { return base == nb ? rem : 0u; }
+    // a bit for each size of pass that there is
+    WL_MEM uint32_t sizes() const { return np == 0u ? 0u : 1u << base | (rem ? 2u << base : 0u); }
 };
 WL_DEV PassSplit pass_split(uint32_t c) {
     const uint32_t m = cdiv(c, kRB), np = cdiv(m, kWide);
@@ -363,7 +365,7 @@ WL_DEV PassSplit pass_split(uint32_t c) {
 // E counts the MXFP4 shared pseudo-expert (index E - 1) when there is one:
 // all T tokens, compact rows from T*K on.
 struct ExpertTab {
-    uint32_t *cnt, *off, *pp;
+    uint32_t *cnt, *off, *pp, *sizes;  // (sizes: each wave's bits of the pass sizes of its experts)
 };
 // Pass table of the passes of nb row blocks: pp the exclusive prefix of the
 // experts' passes, pp[E] all of them (rewritten for each nb). Units are numbered
@@ -466,7 +468,7 @@ WL_DEV void fill_tokens(const Kn& k, uint16_t* tt, uint32_t W) {
                 for (uint32_t j = 0; j < M; j++) {
                     const uint32_t m = lane + 64u * j;
                     has[r][j] = x.live && x.e != k.a.E && m < x.nt;
-                    if (has[r][j]) ent[r][j] = k.ent ? (uint32_t)k.ent[x.row0 + m] : k.b.ent[x.row0 + m];
+                    if (has[r][j]) ent[r][j] = k.b.ent[x.row0 + m];
                 }
             }
         }
@@ -647,8 +649,8 @@ int launch_batched(const DecodeArgs* d_args, const BatchArgs& b, uint32_t H, uin
     bt.tcap = batched_tok_entries(b.T, I, E, K, n_cu);
     const size_t room = (size_t)decode_max_lds() - 3u * (size_t)kSlotB;
     bt.group = phases == kPhaseAll && !(b.flags & kBatchSkipUnbound) && b.T * K <= kGroupMax &&
-               ent_table_offset(E, bt.tcap) + 2u * kGroupMax <= room;
-    const size_t up_lds = bt.group ? ent_table_offset(E, bt.tcap) + 2u * kGroupMax : bup_lds(b.T, I, E, K, n_cu);
+               4u * E * group_words(b.T) <= kSlotB && tok_table_offset(E) + 2u * b.T * K <= room;
+    const size_t up_lds = bt.group ? tok_table_offset(E) + 2u * b.T * K : bup_lds(b.T, I, E, K, n_cu);
     if (up_lds + 3u * (size_t)kSlotB > (size_t)decode_max_lds()) return (int)hipErrorInvalidValue;
     const void *up = (const void*)bup_kernel, *down = (const void*)bdown_kernel;
     const struct { const void* fn; size_t lds; } attrs[] = {
