@@ -49,6 +49,24 @@ WL_DEV void pipeline_drain() { step_barrier<0>(); }
 struct UnitInfo {
     bool live;
     uint32_t e, part, nt, row0;
+    uint32_t m0 = 0u, m1 = 4u;  // its slices (gate/up of small passes; others have all four)
+};
+// Which units are a work-group's. The units of a kernel stand in one row, position s:
+// the shared expert's from 0, then the routed passes'. Position s < G is work-group
+// s's, a later one work-group (s + skip) % G's: skip work-groups, those of the shared
+// expert's units, go without one of the second round.
+struct Places {
+    uint32_t base, s0, s1;  // the pipeline's first position, the work-group's first two there
+    WL_MEM static Places from(uint32_t base, uint32_t skip) {
+        const uint32_t G = gridDim.x, b = blockIdx.x, l = b >= skip ? G + b - skip : 2u * G + b - skip;
+        if (base <= b) return Places{base, b, l};
+        const uint32_t s0 = l + (base > l ? cdiv(base - l, G) : 0u) * G;
+        return Places{base, s0, s0 + G};
+    }
+    WL_MEM uint32_t place(uint32_t i) const { return i == 0u ? s0 : s1 + (i - 1u) * gridDim.x; }
+    WL_MEM uint32_t count(uint32_t end) const {  // those below position end
+        return s0 >= end ? 0u : s1 >= end ? 1u : 1u + cdiv(end - s1, gridDim.x);
+    }
 };
 
 // ---- pipeline ------------------------------------------------------------------------
@@ -311,7 +329,7 @@ struct SharedK {
         }
     }
 };
-// Its units start at work-group 0; returns their count.
+// Its units are the first; returns their count.
 template <bool UP, uint32_t NT, uint32_t NB>
 WL_DEV uint32_t run_shared(const DecodeArgs& a, const BatchArgs& b) {
     SharedK<UP, NT, NB> k{a, b};
@@ -435,13 +453,15 @@ struct QBase {
     static_assert(kTileB * kTiles + 8192u <= kSlotB, "a step's tiles fit a slot");
     const DecodeArgs& a;
     const BatchArgs& b;
-    uint32_t H, I, E, K, nk, S, nq, parts, nst, nst2, nu, v, lane, uoff;
+    uint32_t H, I, E, K, nk, S, nq, parts, nst, nst2, nu, v, lane;
+    Places pl;
+    uint32_t tail, cut;  // units from position tail on are cut into 1 << cut
     PassTab pt;
     const uint8_t* const* stab;
     NativeLayout NL;
     Cursor cn, cc;  // positions of the loads and of the compute
     const uint8_t* wbase;  // the weight stream's block and size (see SharedK)
-    uint32_t wbytes, wpart, vw, vs, lo8, lo16;
+    uint32_t wbytes, wpart, wm0, wm1, vw, vs, lo8, lo16;
     UnitInfo cu, un;     // the unit computed, the unit whose loads go out
     // any row of the call has further pieces; the positions of these units among the
     // work-group's, whether they run twice and are in their second run
@@ -453,8 +473,14 @@ struct QBase {
     WL_MEM UnitInfo unit(uint32_t i) const {
         UnitInfo x{false, 0u, 0u, 0u, 0u};
         if (i >= nu) return x;
-        const uint32_t u = (blockIdx.x + gridDim.x - uoff) % gridDim.x + gridDim.x * i;
-        const PassPart jp = pass_part(u, parts, pt.n);
+        uint32_t s = pl.place(i);
+        if (s >= tail) {
+            const uint32_t w = 4u >> cut, p = (s - tail) & ((1u << cut) - 1u);
+            s = tail + ((s - tail) >> cut);
+            x.m0 = p * w;
+            x.m1 = x.m0 + w;
+        }
+        const PassPart jp = pass_part(s - pl.base, parts, pt.n);
         const Pass ps = pass_at(pt, E, jp.j);
         x.live = true;
         x.part = jp.part;
@@ -492,6 +518,8 @@ struct QBase {
         wbase = blk;
         wbytes = blk ? (uint32_t)NL.total : 0u;
         wpart = x.part;
+        wm0 = x.m0;
+        wm1 = x.m1;
         const uint32_t kd = UP ? H : I, n = 8u * (v & 1u) + lane / 8u, c8 = lane % 8u ^ q_swizzle(n);
         const uint32_t nrow = UP ? b.T : b.T * (K + ((b.flags & kBatchShared4) ? 1u : 0u));
         const uint32_t rec = (uint32_t)q6_row_bytes(kd), ext = (uint32_t)q6_more_bytes(kd);
@@ -551,7 +579,8 @@ struct QBase {
         for (uint32_t i = 0; i < 4; i += 2) {
             const uint32_t sl = cu.part * 4u + i + (gg >> 1);
             const f32x4 x = swiglu_pair(d(i), d(i + 1u));
-            if (r < cu.nt && sl < S) gst((f32x4*)(o + sl * kSlice), x);
+            const uint32_t m = i + (gg >> 1);
+            if (r < cu.nt && sl < S && m >= cu.m0 && m < cu.m1) gst((f32x4*)(o + sl * kSlice), x);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
@@ -587,7 +616,8 @@ struct QNarrow : QBase<UP, NB, 2> {
         uint32_t ch;
         if (UP) ch = min(this->wpart * 4u + j / 2u, this->S - 1u) * 8u * this->nk + min(2u * s + j % 2u, this->nk - 1u);
         else ch = min(4u * s + j / 2u, 2u * this->nk - 1u) * this->nq + min(16u * this->wpart + 2u * this->v + j % 2u, this->nq - 1u);
-        W.w[j] = bld16_nt(rs, this->vw, ch * 1024u);
+        const bool has = !UP || NB > 1u || (j / 2u >= this->wm0 && j / 2u < this->wm1);
+        W.w[j] = bld16_nt(rs, has ? this->vw : kOOBV, ch * 1024u);
     }
     WL_MEM void begin(uint32_t i) {
         this->begin_unit(i);
@@ -761,16 +791,15 @@ constexpr uint32_t kGroupMax = 4u * kGT;
 // Words of token bits of an expert; they have to fit a slot.
 __host__ __device__ inline uint32_t group_words(uint32_t T) { return (T + 31u) / 32u; }
 // Afterwards ent[r] is the token of compact entry r (in the place of the token table).
-WL_DEV void group_entries(const BatchArgs& b, uint32_t E, uint32_t K, const ExpertTab& et, uint16_t* ent) {
+// (id: this thread's entries' experts, entry threadIdx.x + kGT r in id[r].)
+WL_DEV void group_entries(const BatchArgs& b, uint32_t E, uint32_t K, const ExpertTab& et, uint16_t* ent,
+                          const uint32_t (&id)[kGroupMax / kGT]) {
     constexpr uint32_t N = kGroupMax / kGT;
     const uint32_t n = b.T * K, i = threadIdx.x, lane = i & 63u, nw = group_words(b.T);
     uint32_t* bits = (uint32_t*)slot<0>();  // (free until the first pipeline)
-    uint32_t id[N], t[N], rank[N];
+    uint32_t t[N], rank[N];
 #pragma unroll
-    for (uint32_t r = 0; r < N; r++) {
-        t[r] = (i + r * kGT) / K;
-        id[r] = i + r * kGT < n ? (uint32_t)gld(b.idx + i + r * kGT) : 0u;
-    }
+    for (uint32_t r = 0; r < N; r++) t[r] = (i + r * kGT) / K;
     for (uint32_t f = i; f < E * nw; f += kGT) bits[f] = 0u;
     lds_barrier();
 #pragma unroll
@@ -826,14 +855,15 @@ WL_DEV void group_entries(const BatchArgs& b, uint32_t E, uint32_t K, const Expe
     }
     if (i == 0u) gst(b.offsets + E, n);
 }
+template <bool UP>
 WL_DEV ExpertTab load_expert_tab(const BatchArgs& b, uint32_t E, uint32_t K, uint32_t* s, const uint8_t* const* stab,
-                                 bool up) {
-    const ExpertTab et{s, s + E, s + 2u * E, s + 3u * E + 1u};
+                                 const uint32_t (&ids)[kGroupMax / kGT]) {
+    const ExpertTab et{s, s + E, s + 2u * E, s + 3u * E + 1u, s + 3u * E + 1u + kGW};
     const bool skip = (b.flags & kBatchSkipUnbound) != 0u;
     const uint32_t esh = (b.flags & kBatchShared4) ? E - 1u : E;
-    const bool group = up && b.group != 0u;
-    if (group) group_entries(b, esh, K, et, (uint16_t*)(dyn_lds() + tok_table_offset(esh)));
-    uint32_t sizes = 0;
+    const bool group = UP && b.group != 0u;
+    if (group) group_entries(b, esh, K, et, (uint16_t*)(dyn_lds() + tok_table_offset(esh)), ids);
+    uint32_t sizes = 0, sums = 0;
     for (uint32_t f = threadIdx.x; f < E; f += kGT) {
         uint32_t c;
         if (f == esh) {
@@ -847,20 +877,27 @@ WL_DEV ExpertTab load_expert_tab(const BatchArgs& b, uint32_t E, uint32_t K, uin
             et.off[f] = gld(b.offsets + f);
         }
         et.cnt[f] = c;
-        sizes |= pass_split(c).sizes();
+        const PassSplit sp = pass_split(c, false);
+        sizes |= sp.sizes();
+        sums += sp.np + ((cdiv(c, kRB) - sp.np) << 16);
     }
 #pragma unroll
-    for (uint32_t o = 1; o < 64u; o <<= 1) sizes |= __shfl_xor(sizes, (int)o, 64);
-    if ((threadIdx.x & 63u) == 0u) et.sizes[threadIdx.x >> 6] = sizes;
+    for (uint32_t o = 1; o < 64u; o <<= 1) {
+        sizes |= __shfl_xor(sizes, (int)o, 64);
+        sums += __shfl_xor(sums, (int)o, 64);
+    }
+    if ((threadIdx.x & 63u) == 0u) {
+        et.sizes[threadIdx.x >> 6] = sizes;
+        et.sums[threadIdx.x >> 6] = sums;
+    }
     return et;
 }
-// The routed passes of NB row blocks, starting at work-group uoff; returns
-// their units' count.
+// The routed passes of NB row blocks at pl; returns their units' count.
 template <bool UP, uint32_t NB>
 WL_DEV uint32_t run_routed(const DecodeArgs& a, const BatchArgs& b, uint32_t E, const ExpertTab& et,
-                           const uint8_t* const* stab, uint32_t uoff, bool any) {
+                           const uint8_t* const* stab, Places pl, bool any, bool single) {
     using Kn = std::conditional_t<(NB > 2u), QWide<UP, NB>, QNarrow<UP, NB>>;
-    const PassTab pt = load_pass_tab(et, E, NB);
+    const PassTab pt = load_pass_tab(et, E, NB, single);
     pipeline_drain();
     const uint32_t H = a.H, I = a.I;
     Kn w(a, b);
@@ -874,10 +911,20 @@ WL_DEV uint32_t run_routed(const DecodeArgs& a, const BatchArgs& b, uint32_t E, 
     w.parts = UP ? cdiv(w.S, 4u) : cdiv(w.nq, 16u);
     w.nst2 = cdiv(UP ? H : I, 256u);
     w.nst = NB > 2u ? w.nk : w.nst2;
-    w.uoff = uoff % gridDim.x;
-    const uint32_t U = pt.n * w.parts, b0 = (blockIdx.x + gridDim.x - w.uoff) % gridDim.x;
+    const uint32_t U = pt.n * w.parts, end = pl.base + U, G = gridDim.x;
     w.any = any;
-    w.nu = U > b0 ? cdiv(U - b0, gridDim.x) : 0u;
+    w.pl = pl;
+    // gate/up of one row block: the units of the last round, where at most half of
+    // the work-groups have one, go to two or four of them each (not with a token table:
+    // it is sized for cdiv(U, G) units of a work-group)
+    w.tail = end;
+    w.cut = 0u;
+    if (UP && NB == 1u && b.group && end > G) {
+        const uint32_t rem = (end - G) % G;
+        w.cut = rem == 0u || rem > U || 2u * rem > G ? 0u : 4u * rem > G ? 1u : 2u;
+        if (w.cut) w.tail = end - rem;
+    }
+    w.nu = pl.count(w.tail + ((end - w.tail) << w.cut));
     w.lane = threadIdx.x & 63u;
     w.v = uni(threadIdx.x >> 6);
     w.lo8 = q_lo8();
@@ -908,20 +955,43 @@ WL_DEV void run_gemm(const DecodeArgs* pa, const BatchArgs& b) {
     const DecodeArgs& a = *pa;
     uint8_t* dyn = dyn_lds();
     const bool sh4 = (b.flags & kBatchShared4) != 0u;
-    const bool any = uni(gld(b.more + (UP ? 0 : 1))) != 0u;
+    // (the loads of the tables go out together, as their waits are the head of the
+    // kernel)
+    const uint32_t more = gld(b.more + (UP ? 0 : 1));
+    uint32_t ids[kGroupMax / kGT];
+    if (UP && b.group) {
+#pragma unroll
+        for (uint32_t r = 0; r < kGroupMax / kGT; r++)
+            ids[r] = (uint32_t)gld(b.idx + min(threadIdx.x + r * kGT, b.T * a.K - 1u));
+    }
     const uint32_t E = a.E + (sh4 ? 1u : 0u);  // experts in the pass table
     const uint8_t* const* stab = load_slot_tab(a, a.E, sh4, (const uint8_t**)dyn);
-    const ExpertTab et = load_expert_tab(b, E, a.K, (uint32_t*)(dyn + 8u * E), stab, UP);
+    const ExpertTab et = load_expert_tab<UP>(b, E, a.K, (uint32_t*)(dyn + 8u * E), stab, ids);
     uint32_t u = run_shared_expert<UP>(a, b);
+    // (a pass over more than 32 tokens takes one and a half to two times a routed unit:
+    // 80 tokens 804 to 791 us, 96 841 to 828; past 128 there are too many)
+    const uint32_t skip = b.T > 32u && b.T <= 128u && u < gridDim.x && (!UP || b.group) ? u : 0u;
     // (pass sizes that no expert has cost a table of 2 us each where they were
     // looked up one by one)
     lds_barrier();
-    uint32_t sizes = 0;
+    uint32_t sizes = 0, sums = 0;
 #pragma unroll
-    for (uint32_t w = 0; w < kGW; w++) sizes |= et.sizes[w];
+    for (uint32_t w = 0; w < kGW; w++) {
+        sizes |= et.sizes[w];
+        sums += et.sums[w];
+    }
     sizes = uni(sizes);
-    if (sizes & 1u << 4) u += run_routed<UP, 4>(a, b, E, et, stab, u, any);
-    if (sizes & 1u << 3) u += run_routed<UP, 3>(a, b, E, et, stab, u, any);
-    if (sizes & 1u << 2) u += run_routed<UP, 2>(a, b, E, et, stab, u, any);
-    if (sizes & 1u << 1) run_routed<UP, 1>(a, b, E, et, stab, u, any);
+    sums = uni(sums);
+    // Few larger passes among many small ones run as passes of one block, if that adds
+    // at most a 64th to the weights read: a pipeline of their own, a unit or two for
+    // some of the work-groups, had these end last (at 64 tokens, one expert of two
+    // blocks among 213: by 17 us of 465, bdown 28 of 271). (Not with a token table,
+    // which is sized for one small pass per expert.)
+    const bool single = sums >> 16 != 0u && 64u * (sums >> 16) <= (sums & 0xFFFFu) && (!UP || b.group);
+    if (single) sizes = 2u;
+    const bool any = uni(more) != 0u;
+    if (sizes & 1u << 4) u += run_routed<UP, 4>(a, b, E, et, stab, Places::from(u, skip), any, single);
+    if (sizes & 1u << 3) u += run_routed<UP, 3>(a, b, E, et, stab, Places::from(u, skip), any, single);
+    if (sizes & 1u << 2) u += run_routed<UP, 2>(a, b, E, et, stab, Places::from(u, skip), any, single);
+    if (sizes & 1u << 1) run_routed<UP, 1>(a, b, E, et, stab, Places::from(u, skip), any, single);
 }

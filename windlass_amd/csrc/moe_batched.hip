@@ -357,15 +357,18 @@ struct PassSplit {
     // a bit for each size of pass that there is
     WL_MEM uint32_t sizes() const { return np == 0u ? 0u : 1u << base | (rem ? 2u << base : 0u); }
 };
-WL_DEV PassSplit pass_split(uint32_t c) {
-    const uint32_t m = cdiv(c, kRB), np = cdiv(m, kWide);
-    return np == 0u ? PassSplit{0u, 0u, 0u} : PassSplit{np, m / np, m % np};
+// (single: into passes of one block)
+WL_DEV PassSplit pass_split(uint32_t c, bool single) {
+    const uint32_t m = cdiv(c, kRB), np = single ? m : cdiv(m, kWide);
+    if (np <= 1u) return PassSplit{np, m, 0u};  // (most: no division)
+    return PassSplit{np, m / np, m % np};
 }
 // The experts' counts and offsets, in LDS, and room for the pass table.
 // E counts the MXFP4 shared pseudo-expert (index E - 1) when there is one:
 // all T tokens, compact rows from T*K on.
 struct ExpertTab {
-    uint32_t *cnt, *off, *pp, *sizes;  // (sizes: each wave's bits of the pass sizes of its experts)
+    uint32_t *cnt, *off, *pp;
+    uint32_t *sizes, *sums;  // each wave's, of its experts: bits of the sizes of their passes; passes | more if single << 16
 };
 // Pass table of the passes of nb row blocks: pp the exclusive prefix of the
 // experts' passes, pp[E] all of them (rewritten for each nb). Units are numbered
@@ -375,15 +378,16 @@ struct ExpertTab {
 struct PassTab {
     const uint32_t *cnt, *off, *pp;
     uint32_t n, nb;  // passes; row blocks of each
+    bool single;
 };
-WL_DEV PassTab load_pass_tab(const ExpertTab& et, uint32_t E, uint32_t nb) {
+WL_DEV PassTab load_pass_tab(const ExpertTab& et, uint32_t E, uint32_t nb, bool single) {
     const uint32_t tid = threadIdx.x;
     lds_barrier();  // the tables are written, the last pass table is no longer read
     if (tid < 64u) {
         const uint32_t per = cdiv(E, 64u), e0 = tid * per;
         uint32_t mine = 0;
         for (uint32_t i = 0; i < per; i++)
-            if (e0 + i < E) mine += pass_split(et.cnt[e0 + i]).count(nb);
+            if (e0 + i < E) mine += pass_split(et.cnt[e0 + i], single).count(nb);
         uint32_t inc = mine;
 #pragma unroll
         for (uint32_t o = 1; o < 64u; o <<= 1) {
@@ -394,12 +398,12 @@ WL_DEV PassTab load_pass_tab(const ExpertTab& et, uint32_t E, uint32_t nb) {
         for (uint32_t i = 0; i < per; i++)
             if (e0 + i < E) {
                 et.pp[e0 + i] = run;
-                run += pass_split(et.cnt[e0 + i]).count(nb);
+                run += pass_split(et.cnt[e0 + i], single).count(nb);
             }
         if (tid == 63u) et.pp[E] = inc;
     }
     lds_barrier();
-    return PassTab{et.cnt, et.off, et.pp, uni(et.pp[E]), nb};
+    return PassTab{et.cnt, et.off, et.pp, uni(et.pp[E]), nb, single};
 }
 // Routed unit r (< n_passes * parts) -> (pass j, part). Units go in blocks
 // of 8 passes x parts, ordered so that unit r has j % 8 == r % 8 in full
@@ -432,7 +436,7 @@ WL_DEV uint32_t expert_of_pass(const uint32_t* pp, uint32_t E, uint32_t j) {
 }
 WL_DEV Pass pass_at(const PassTab& pt, uint32_t E, uint32_t j) {
     const uint32_t e = expert_of_pass(pt.pp, E, j), c = uni(pt.cnt[e]);
-    const PassSplit sp = pass_split(c);
+    const PassSplit sp = pass_split(c, pt.single);
     const uint32_t p = sp.first(pt.nb) + j - uni(pt.pp[e]), r0 = kRB * (p * sp.base + min(p, sp.rem));
     return Pass{e, min(kRB * pt.nb, c - r0), uni(pt.off[e]) + r0};
 }
