@@ -2,8 +2,7 @@
 
 A block of 32 activations shares its scales (csrc/q6.h), so one value far above
 the others may not cost them their bits. One to three columns of every second
-block of the normalised input (at the largest ratio sixteen of the last block) are
-`ratio` times the others, and every expert's
+block of the normalised input are `ratio` times the others, and every expert's
 gate and up weights are zero there; some rows of gate and up make SwiGLU values
 about `ratio` times the others, and down is zero there. What comes out then is made
 by the outliers' neighbours alone. All tokens go to the same experts, so passes of
@@ -34,10 +33,6 @@ MID_COLS = [32 * b + 11 for b in range(0, I // 32, 2)]
 BAR = 1.1e-6
 
 
-def _in_cols(ratio):
-    return IN_COLS + ([H - 32 + 2 * i for i in range(16)] if ratio == 30000 else [])
-
-
 def _zero_columns(nib, cols):
     for c in cols:
         nib[:, c // 2] &= np.uint8(0xF0 if c % 2 == 0 else 0x0F)
@@ -46,7 +41,7 @@ def _zero_columns(nib, cols):
 def _block(e, ratio):
     gw, gs, uw, us, dw, ds = [a.copy() for a in synth.expert_block(H, I, SEED, 0, e)]
     for w in (gw, uw):
-        _zero_columns(w, _in_cols(ratio))
+        _zero_columns(w, IN_COLS)
     _zero_columns(dw, MID_COLS)
     up = int(round(np.log2(ratio) / 2))  # the product of gate and up
     gs[MID_COLS] += np.uint8(up + 3)     # (silu is g / 2 near zero)
@@ -83,11 +78,10 @@ def test_neighbours_of_outliers_keep_their_bits(gpu, ratio):
             (dense["router_w"], bias, np.concatenate([p.reshape(-1) for p in shared]))]
     ctx.set_layer(0, bufs[0].ptr, bufs[1].ptr, None, bufs[2].ptr, moe.SHARED_MXFP4)
     worst = {}
-    cols = _in_cols(ratio)
     for T in (3, 16, 20, 40, 64, 70, 150):
         for step in (1, 2):
             hs = np.stack([synth.hidden_state(H, 4100 + T, t) for t in range(T)]).astype(np.float32)
-            hs[step - 1::step, cols] *= np.float32(ratio)
+            hs[step - 1::step, IN_COLS] *= np.float32(ratio)
             x, o = H_.DeviceBuffer.from_array(hs), H_.DeviceBuffer(4 * T * H)
             ctx.run_moe_batched(0, T, x.ptr, None, o.ptr)
             ctx.check_error()

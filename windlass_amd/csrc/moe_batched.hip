@@ -250,10 +250,11 @@ __global__ void __launch_bounds__(kThreads) btopk_kernel(const DecodeArgs* __res
     const DecodeArgs& a = *pa;
     const uint32_t H = a.H, E = a.E, K = a.K, t = blockIdx.x, tid = threadIdx.x;
     __shared__ __align__(16) float row[(8192 / 32) * 36];  // 4 floats between blocks of 32: other banks
-    __shared__ uint32_t more;
+    __shared__ uint32_t wide;
+    __shared__ double part[2][kWaves];
     float* rowp = b.norm + (size_t)t * b.ldn;
     for (uint32_t j = tid; j < H / 4u; j += kThreads) *(u32x4*)(row + 36u * (j / 8u) + 4u * (j % 8u)) = gld16(rowp + 4u * j);
-    if (tid == 0u) more = 0u;
+    if (tid == 0u) wide = 0u;
     extern __shared__ __align__(16) uint8_t lds[];
     float* tk_sc = (float*)lds;
     float* tk_ch = tk_sc + E;
@@ -263,11 +264,13 @@ __global__ void __launch_bounds__(kThreads) btopk_kernel(const DecodeArgs* __res
         topk_score(gld(b.logits + (size_t)t * E + e), gld(a.bias + e), e, tk_sc, tk_ch);
     lds_barrier();  // (every thread's reads of the row are done)
     f32x16 even, odd;
+    QRange rg{0.0, 0.0, false};
     auto quantise = [&](uint32_t i) {
         if (i >= H / 32u) return;
         q6_load(row + 36u * i, even, odd);
         const uint32_t mx = q6_max(even, odd);
-        if (q6_wide(even, odd, mx)) more = 1u;
+        rg = q6_range(even, odd, mx);
+        if (rg.wide) wide = 1u;
         q6_store<false>((uint8_t*)rowp + (i / 4u) * kQRecord, i % 4u, even, odd, mx);
     };
     // up to 256 experts the argmax is wave 0's: the other waves quantise (at most
@@ -284,8 +287,23 @@ __global__ void __launch_bounds__(kThreads) btopk_kernel(const DecodeArgs* __res
         gst(b.idx + (size_t)t * K + tid, (int32_t)tk_idx[tid]);
         gst(b.wts + (size_t)t * K + tid, topk_weight(a, K, tk_w, tid));
     }
-    if (tid == 0u) gst(b.more_up + t, more);
-    if (more == 0u) return;
+    bool more = false;
+    if (wide != 0u) {
+        const double big = wave_sum_f64(rg.big), rest = wave_sum_f64(rg.rest);
+        if ((tid & 63u) == 0u) {
+            part[0][tid >> 6] = big;
+            part[1][tid >> 6] = rest;
+        }
+        lds_barrier();
+        double sb = 0.0, sr = 0.0;
+        for (uint32_t w = 0; w < kWaves; w++) {
+            sb += part[0][w];
+            sr += part[1][w];
+        }
+        more = q6_more(sb, sr);
+    }
+    if (tid == 0u) gst(b.more_up + t, more ? 1u : 0u);
+    if (!more) return;
     if (tid == 0u) gst(b.more, 1u);
     if (tid < H / 32u) {
         q6_load(row + 36u * tid, even, odd);
@@ -541,6 +559,7 @@ __global__ void __launch_bounds__(256) bquant_kernel(const DecodeArgs* __restric
     const float* mid = b.midf + (size_t)min(row, R - 1u) * b.ldm;
     f32x16 even, odd;
     bool wide = false;
+    double big = 0.0, rest = 0.0;
     for (uint32_t b0 = 0; b0 < nb; b0 += 64u) {
 #pragma unroll
         for (uint32_t i = 0; i < 8; i++) {
@@ -552,12 +571,16 @@ __global__ void __launch_bounds__(256) bquant_kernel(const DecodeArgs* __restric
         if (row < R && k < nb) {
             q6_load(xs[v] + 36u * lane, even, odd);
             const uint32_t mx = q6_max(even, odd);
-            wide |= q6_wide(even, odd, mx);
+            const QRange rg = q6_range(even, odd, mx);
+            wide |= rg.wide;
+            big += rg.big;
+            rest += rg.rest;
             q6_store<false>(b.mid6 + (size_t)row * q6_row_bytes(I) + (k / 4u) * kQRecord, k % 4u, even, odd, mx);
         }
         lds_barrier();
     }
-    const bool more = __builtin_amdgcn_ballot_w64(wide) != 0u;
+    bool more = false;
+    if (__builtin_amdgcn_ballot_w64(wide) != 0u) more = q6_more(wave_sum_f64(big), wave_sum_f64(rest));
     if (row < R && lane == 0u) {
         gst(b.more_dn + row, more ? 1u : 0u);
         if (more) gst(b.more + 1, 1u);

@@ -13,19 +13,21 @@
 // it, 21 bits down to 1/256.
 //
 // That is enough for a block whose values are of one size. Where most lie far below
-// a few (q6_wide), as beside the outlier channels of a trained model, weights that
-// are zero at those few (MXFP4 rounds many to zero) leave a sum of the small ones
-// alone; with five pieces such sums were off by 3e-6 of the largest output at 100
-// times, 1e-3 at 30000 times, and six leave a 32nd of that. A row with such a block
-// therefore has two further pieces per block, in records of their own that the GEMMs
-// run as a second pass over the same weights, into the same sums: 2^-39 of the
-// largest value, full f32 precision down to 1/32768 of it. The test counts values
-// rather than looking at the smallest: SwiGLU values are products, and some of any
-// 32 are small. Normal inputs and the SwiGLU values they make take none (4096 tokens
-// of hidden 6144). Units with such rows run twice as long (hidden 6144, inter 2048, 8
+// a few, as beside the outlier channels of a trained model, weights that are zero at
+// those few (MXFP4 rounds many to zero) leave a sum of the small ones alone; with five
+// pieces such sums were off by 3e-6 of the largest output at 100 times, 1e-3 at 30000
+// times, and six leave a 32nd of that. A row in which this may count therefore has two
+// further pieces per block, in records of their own that the GEMMs run as a second
+// pass over the same weights, into the same sums: 2^-39 of the largest value, full
+// f32 precision down to 1/32768 of it. It counts where what six pieces leave of the
+// wide blocks, some 2^-31 of the largest for each of 32 values, may exceed 2^-24.5 of
+// the row's sum without their few large values (q6_more). The row's other blocks are in
+// that sum: SwiGLU values of large gate values, half of them almost zero, make many
+// blocks wide and lose nothing (a rule block by block took further pieces for them and
+// 64 tokens 755 to 940 us). Units with such rows run twice as long (hidden 6144, inter 2048, 8
 // of 256 experts, 12 columns 1000 times the rest in one token, or in every one: 7
-// tokens 247 and 306 us, without 214; 1000 tokens 1646 and 2290, 1601; 4096 tokens
-// 5263 and 7135, 5180).
+// tokens 241 and 299 us, without 207; 1000 tokens 1690 and 2335, 1625; 4096 tokens
+// 5347 and 7304, 5260).
 //
 // Why this format: measured on MI355X the instruction runs 8.5 PFLOP/s with 6-bit
 // against 4-bit operands (bf16 2.43, 8-bit 4.8), so six pieces cost 0.6 of three
@@ -78,20 +80,41 @@ WL_DEV uint32_t q6_max(const f32x16& even, const f32x16& odd) {
     }
     return mx;
 }
-// Whether a block of largest magnitude mx takes further pieces: at most eight of
-// its values are within 2^8 of the largest and smaller ones are there, or twelve lie
-// under 2^-12 of it.
-WL_DEV bool q6_wide(const f32x16& even, const f32x16& odd, uint32_t mx) {
-    const float m = __uint_as_float(mx), lim = m * 0x1p-8f, lim2 = m * 0x1p-12f;
-    uint32_t large = 0u, zero = 0u, tiny = 0u;
+// What a block of largest magnitude mx adds to its row's test for further pieces
+// (q6_more). big: the square of the largest value if the block is wide, that is at most
+// eight of its values are within 2^8 of the largest and smaller ones are there. rest:
+// the sum of squares of those smaller ones; in other blocks that of the values under an
+// eighth of the largest, if at most eight reach that (outliers, too), or of all.
+struct QRange {
+    double big, rest;
+    bool wide;
+};
+WL_DEV QRange q6_range(const f32x16& even, const f32x16& odd, uint32_t mx) {
+    const float m = __uint_as_float(mx), inv = __builtin_amdgcn_rcpf(m);
+    float all = 0.f, s3 = 0.f, s8 = 0.f;
+    uint32_t n3 = 0u, n8 = 0u, zero = 0u;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const float a = fabsf(even[i]), b = fabsf(odd[i]);
-        large += (a >= lim ? 1u : 0u) + (b >= lim ? 1u : 0u);
-        zero += (a == 0.f ? 1u : 0u) + (b == 0.f ? 1u : 0u);
-        tiny += (a < lim2 ? 1u : 0u) + (b < lim2 ? 1u : 0u);
+    for (int i = 0; i < 32; i++) {
+        const float a = fabsf(i & 1 ? odd[i / 2] : even[i / 2]) * inv, q = a * a;
+        const bool l3 = a >= 0x1p-3f, l8 = a >= 0x1p-8f;
+        all += q;
+        s3 += l3 ? 0.f : q;
+        s8 += l8 ? 0.f : q;
+        n3 += l3 ? 1u : 0u;
+        n8 += l8 ? 1u : 0u;
+        zero += a == 0.f ? 1u : 0u;
     }
-    return mx < 0x7F800000u && ((large <= 8u && large + zero < 32u) || tiny >= zero + 12u);
+    if (m < 0x1p-100f || !(m < INFINITY)) return QRange{0.0, 0.0, false};
+    const bool wide = n8 <= 8u && n8 + zero < 32u;
+    const double m2 = (double)m * (double)m;
+    return QRange{wide ? m2 : 0.0, m2 * (wide ? s8 : n3 <= 8u ? s3 : all), wide};
+}
+// From the row's sums.
+WL_DEV bool q6_more(double big, double rest) { return big > 256.0 * rest; }
+// The sum over a wave.
+WL_DEV double wave_sum_f64(double x) {
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+    return x;
 }
 // Block g of a k tile: 32 values (even[i], odd[i] columns 2i and 2i + 1) of largest
 // magnitude mx into its parts of the record at rec, or (MORE) its further pieces
