@@ -119,6 +119,28 @@ def test_batched_through_source_equals_resident(gpu, shape, native, T):
     dm.close()
 
 
+@pytest.mark.parametrize("shape,T", [("glm", 64), ("glm", 96), ("small", 40)])
+def test_batched_groups_with_mxfp4_shared_equal_resident(gpu, shape, T):
+    """Several groups of experts with an MXFP4 shared expert, which runs with the
+    first: the same bits as the resident layer, whose one launch sees all experts'
+    counts. At the GLM shape one or two of some 210 to 240 experts have more than 16
+    tokens: the passes of few larger experts are cut by all experts' counts, not a
+    group's. Called twice: nothing of the first call is left for the second."""
+    c = GLM if shape == "glm" else SMALL
+    zipf = synthdata.zipf_bias_offset(c["n_routed_experts"], 36, amplitude=0.25)
+    dm = DeviceModel(c, seed=36, n_layers=1, bias_offset=zipf, shared_mxfp4=True)
+    sm = SourceModel(dm)
+    for call in range(2):
+        hs = np.stack([synth.hidden_state(c["hidden"], 820 + call, t) for t in range(T)]).astype(np.float32)
+        got, ref = _batched(sm, hs), _batched(dm, hs)
+        counts = dm.ctx.batched_counts()
+        print(f"{shape} T={T}: {(counts > 0).sum()} experts, {(counts > 16).sum()} of more than 16 tokens", flush=True)
+        assert (counts > 0).sum() > 32
+        assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+    sm.close()
+    dm.close()
+
+
 def test_batched_through_cache_equals_resident(gpu):
     """The built-in cache as the batched layer's source: bit-identical to the
     resident layer, each unique expert requested once."""

@@ -866,19 +866,22 @@ WL_DEV ExpertTab load_expert_tab(const BatchArgs& b, uint32_t E, uint32_t K, uin
     uint32_t sizes = 0, sums = 0;
     for (uint32_t f = threadIdx.x; f < E; f += kGT) {
         uint32_t c;
+        bool here = true;  // its passes are this launch's
         if (f == esh) {
-            c = (b.flags & kBatchNoShared) ? 0u : b.T;
+            c = b.T;
+            here = !(b.flags & kBatchNoShared);
             et.off[f] = b.T * K;
         } else if (group) {
             c = et.cnt[f];
         } else {
             // stab[f] was written by this thread (load_slot_tab, same stride)
-            c = skip && stab[f] == nullptr ? 0u : gld(b.counts + f);
+            c = gld(b.counts + f);
+            here = !skip || stab[f] != nullptr;
             et.off[f] = gld(b.offsets + f);
         }
-        et.cnt[f] = c;
+        et.cnt[f] = here ? c : 0u;
         const PassSplit sp = pass_split(c, false);
-        sizes |= sp.sizes();
+        if (here) sizes |= sp.sizes();
         sums += sp.np + ((cdiv(c, kRB) - sp.np) << 16);
     }
 #pragma unroll
@@ -985,10 +988,10 @@ WL_DEV void run_gemm(const DecodeArgs* pa, const BatchArgs& b) {
     // Few larger passes among many small ones run as passes of one block, if that adds
     // at most a 64th to the weights read: a pipeline of their own, a unit or two for
     // some of the work-groups, had these end last (at 64 tokens, one expert of two
-    // blocks among 213: by 17 us of 465, bdown 28 of 271). (Not with a token table,
-    // which is sized for one small pass per expert.)
-    const bool single = sums >> 16 != 0u && 64u * (sums >> 16) <= (sums & 0xFFFFu) && (!UP || b.group);
-    if (single) sizes = 2u;
+    // blocks among 213: by 17 us of 465, bdown 28 of 271). All experts of the call
+    // count, so that one whose experts come in groups gives the same bits.
+    const bool single = sums >> 16 != 0u && 64u * (sums >> 16) <= (sums & 0xFFFFu);
+    if (single && sizes) sizes = 2u;
     const bool any = uni(more) != 0u;
     if (sizes & 1u << 4) u += run_routed<UP, 4>(a, b, E, et, stab, Places::from(u, skip), any, single);
     if (sizes & 1u << 3) u += run_routed<UP, 3>(a, b, E, et, stab, Places::from(u, skip), any, single);

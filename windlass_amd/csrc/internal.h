@@ -316,6 +316,7 @@ struct BatchArgs {
     float* shout;          // [T][H]
     uint32_t tcap;         // token-table entries per work-group in bup_kernel's LDS (set by launch_batched)
     uint32_t group;        // bup_kernel groups the entries by expert itself (set by launch_batched)
+    uint32_t q0, qn;       // kBatchSkipUnbound: the compact rows of the experts whose blocks are there
 };
 
 // Launchers (moe_decode.hip).

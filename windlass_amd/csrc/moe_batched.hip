@@ -386,7 +386,9 @@ WL_DEV PassSplit pass_split(uint32_t c, bool single) {
 // all T tokens, compact rows from T*K on.
 struct ExpertTab {
     uint32_t *cnt, *off, *pp;
-    uint32_t *sizes, *sums;  // each wave's, of its experts: bits of the sizes of their passes; passes | more if single << 16
+    // each wave's, of its experts: bits of the sizes of this launch's passes; all
+    // passes of the call | more of them if single << 16
+    uint32_t *sizes, *sums;
 };
 // Pass table of the passes of nb row blocks: pp the exclusive prefix of the
 // experts' passes, pp[E] all of them (rewritten for each nb). Units are numbered
@@ -550,13 +552,25 @@ __global__ void __launch_bounds__(kGT) bdown_kernel(const DecodeArgs* __restrict
 
 // The routed SwiGLU values (midf) as quantised rows (mid6, mid6x): a row per wave,
 // one block of 32 values per lane, staged through LDS so that the loads are
-// coalesced.
+// coalesced. Bound by the bytes (4096 tokens of inter 2048, 8 experts each: 590 MB in
+// 112 us); where the experts come in groups, a group's rows and, with the first, the
+// MXFP4 shared expert's alone (quant_rows).
+struct QuantRows {
+    uint32_t q0, qn, n;  // qn rows from q0, then the shared expert's (from T K on), n in all
+};
+__host__ __device__ inline QuantRows quant_rows(const BatchArgs& b, uint32_t K) {
+    const bool part = (b.flags & kBatchSkipUnbound) != 0u;
+    const uint32_t qn = part ? b.qn : b.T * K, sh = (b.flags & kBatchShared4) && !(b.flags & kBatchNoShared) ? b.T : 0u;
+    return QuantRows{part ? b.q0 : 0u, qn, qn + sh};
+}
 __global__ void __launch_bounds__(256) bquant_kernel(const DecodeArgs* __restrict__ pa, const BatchArgs b) {
     const DecodeArgs& a = *pa;
     const uint32_t I = a.I, nb = I / 32u, lane = threadIdx.x & 63u, v = uni(threadIdx.x >> 6);
-    const uint32_t R = b.T * (a.K + ((b.flags & kBatchShared4) ? 1u : 0u)), row = blockIdx.x * 4u + v;
+    const QuantRows qr = quant_rows(b, a.K);
+    const uint32_t i0 = min(blockIdx.x * 4u + v, qr.n - 1u), row = i0 < qr.qn ? qr.q0 + i0 : b.T * a.K + i0 - qr.qn;
+    const bool live = blockIdx.x * 4u + v < qr.n;
     __shared__ __align__(16) float xs[4][64 * 36];  // 32 values + 4: consecutive blocks in different banks
-    const float* mid = b.midf + (size_t)min(row, R - 1u) * b.ldm;
+    const float* mid = b.midf + (size_t)row * b.ldm;
     f32x16 even, odd;
     bool wide = false;
     double big = 0.0, rest = 0.0;
@@ -568,7 +582,7 @@ __global__ void __launch_bounds__(256) bquant_kernel(const DecodeArgs* __restric
         }
         lds_barrier();
         const uint32_t k = b0 + lane;
-        if (row < R && k < nb) {
+        if (live && k < nb) {
             q6_load(xs[v] + 36u * lane, even, odd);
             const uint32_t mx = q6_max(even, odd);
             const QRange rg = q6_range(even, odd, mx);
@@ -581,11 +595,11 @@ __global__ void __launch_bounds__(256) bquant_kernel(const DecodeArgs* __restric
     }
     bool more = false;
     if (__builtin_amdgcn_ballot_w64(wide) != 0u) more = q6_more(wave_sum_f64(big), wave_sum_f64(rest));
-    if (row < R && lane == 0u) {
+    if (live && lane == 0u) {
         gst(b.more_dn + row, more ? 1u : 0u);
         if (more) gst(b.more + 1, 1u);
     }
-    if (row >= R || !more) return;
+    if (!live || !more) return;
     for (uint32_t k = lane; k < nb; k += 64u) {
         q6_load(mid + 32u * k, even, odd);
         q6_store<true>(b.mid6x + (size_t)row * q6_more_bytes(I) + (k / 4u) * kQMore, k % 4u, even, odd, q6_max(even, odd));
@@ -629,15 +643,16 @@ __global__ void __launch_bounds__(256) bcomb_kernel(const BatchArgs b, uint32_t 
 // Token-table entries a work-group of the gate/up kernel can need for T
 // tokens (an upper bound over every routing): R = T (K + 1) rows (K + 1 counts an
 // MXFP4 shared expert's) make at most R / (16 (nb - 1) + 1) passes of nb row
-// blocks, and at most one of one or two row blocks per expert; a work-group gets
-// at most cdiv(units, grid) of them.
+// blocks, and at most one of one or two row blocks per expert, with a 32nd more where
+// all passes have one block (run_gemm); a work-group gets at most cdiv(units, grid)
+// of them.
 static uint32_t batched_tok_entries(uint32_t T, uint32_t I, uint32_t E, uint32_t K, uint32_t grid) {
     auto cd = [](uint64_t a, uint64_t b) { return (a + b - 1u) / b; };
     const uint64_t R = (uint64_t)T * (K + 1u), NS = cd(I / kSlice, 4u);
     uint64_t most = 0;
     for (uint32_t nb = 1; nb <= kWide; nb++) {
         uint64_t n = R / (kRB * (nb - 1u) + 1u);
-        if (nb <= 2u) n = std::min<uint64_t>(n, E + 1u);
+        if (nb <= 2u) n = std::min<uint64_t>(n, E + 1u + (E + 1u) / 32u + 1u);
         most = std::max(most, cd(n * NS, grid) * kRB * nb);
     }
     return (uint32_t)most;
@@ -708,9 +723,9 @@ int launch_batched(const DecodeArgs* d_args, const BatchArgs& b, uint32_t H, uin
     }
     if (phases & kPhaseGemm) {
         const uint32_t gu = resident(up, up_lds), gd = resident(down, gemm_lds);
-        const uint32_t rows = b.T * (K + ((b.flags & kBatchShared4) ? 1u : 0u));
+        const uint32_t rows = quant_rows(b, K).n;
         hipLaunchKernelGGL(bup_kernel, dim3(gu), dim3(kGT), up_lds, s, d_args, bt);
-        hipLaunchKernelGGL(bquant_kernel, dim3((rows + 3u) / 4u), dim3(256), 0, s, d_args, bt);
+        if (rows) hipLaunchKernelGGL(bquant_kernel, dim3((rows + 3u) / 4u), dim3(256), 0, s, d_args, bt);
         hipLaunchKernelGGL(bdown_kernel, dim3(gd), dim3(kGT), gemm_lds, s, d_args, bt);
     }
     if (phases & kPhaseCombine)

@@ -1263,6 +1263,7 @@ static wl_status batched_source_gemms(wl_ctx* c, uint32_t layer, wl::BatchArgs b
         ech = std::min(ech, c->stage_n);
     }
     if (ech == 0) return fail(c, WL_ERR_STATE, "no room to fetch experts");
+    b.q0 = b.qn = 0;
     for (size_t i = 0; i < uniq.size(); i += ech) {
         const uint32_t n = (uint32_t)std::min<size_t>(ech, uniq.size() - i);
         const int32_t* ids = uniq.data() + i;
@@ -1273,6 +1274,10 @@ static wl_status batched_source_gemms(wl_ctx* c, uint32_t layer, wl::BatchArgs b
         int le = wl::launch_slot_fill(c->d_slot + (size_t)layer * E, E, ids, ptrs, n, s);
         if (le != 0) return hip_fail(c, (hipError_t)le, "slot table fill");
         b.flags = (b.flags & wl::kBatchShared4) | wl::kBatchSkipUnbound | (i == 0 ? 0u : wl::kBatchNoShared);
+        // the compact rows lie in expert order, so a group's follow the last one's
+        b.q0 += b.qn;
+        b.qn = 0;
+        for (uint32_t k = 0; k < n; k++) b.qn += counts[ids[k]];
         le = wl::launch_batched(c->d_largs + layer, b, c->cfg.hidden, c->cfg.moe_inter, c->SI, E,
                                 c->cfg.n_experts_per_tok, (uint32_t)c->n_cu, wl::kPhaseGemm, s);
         if (le != 0) return hip_fail(c, (hipError_t)le, "batched GEMM launch");
