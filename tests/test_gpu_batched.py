@@ -19,6 +19,8 @@ SMALL = dict(hidden=384, moe_inter=256, n_routed_experts=48, n_experts_per_tok=6
              routed_scaling=2.5, rms_eps=1e-5)
 GLM = dict(hidden=6144, moe_inter=2048, n_routed_experts=256, n_experts_per_tok=8, n_shared=1,
            routed_scaling=2.5, rms_eps=1e-5)
+# tokens, larger passes cut into passes of one block, parts of a last unit
+SMALL_CALLS = [(12, False, 2), (16, False, 4), (36, False, 4), (44, True, 1), (56, True, 2), (84, True, 2), (124, True, 4)]
 
 
 def _tokens(H, T, seed):
@@ -263,26 +265,41 @@ def test_calls_longer_than_a_chunk(gpu):
     dm.close()
 
 
-@pytest.mark.parametrize("T", [64, 256])
-def test_small_expert_units_equal_grouped_passes(gpu, monkeypatch, T):
-    """At the GLM shape experts of up to 8 tokens run their gate/up and down
-    as streaming units instead of grouped passes (the kernels' small-expert
-    instantiations). WL_BATCHED_SMALL=0 keeps every
-    expert in the grouped passes; both give the same outputs bit for bit,
-    with the bench's Zipf bias (T = 64: most experts hold 1-4 tokens; 256:
-    most hold 5-16)."""
+def _small_call(counts, T, inter=2048, grid=256):
+    """How the gate/up kernel lays out a small call (csrc/batched_gemm.h, run_gemm and
+    run_routed): whether its few larger passes are cut into passes of one block, and
+    into how many parts the units of its last round are."""
+    m = -(-counts.astype(int) // 16)
+    np_ = -(-m // 4)
+    extra, passes = int((m - np_).sum()), int(np_.sum())
+    single = 0 < 64 * extra <= passes
+    if extra and not single:
+        return single, 1
+    shared = -(-T // 64) * (inter // 64)
+    end = shared + (passes + extra) * -(-(inter // 64) // 4)
+    rem = (end - grid) % grid if end > grid else 0
+    return single, 1 if rem == 0 or 2 * rem > grid else 2 if 4 * rem > grid else 4
+
+
+@pytest.mark.parametrize("T,single,parts", SMALL_CALLS)
+def test_glm_small_batches_vs_decode(gpu, T, single, parts):
+    """GLM-shape calls whose experts nearly all have at most 16 tokens: passes of one
+    block, the few larger ones cut into such, the units of the last round whole or in
+    two or four parts, work-groups of the shared expert's units a round behind. Every
+    token against the decode path, the first and last against the oracle."""
     c = GLM
     H = c["hidden"]
     zipf = synthdata.zipf_bias_offset(c["n_routed_experts"], 1, amplitude=0.25)
     dm = DeviceModel(c, seed=1, n_layers=1, bias_offset=zipf)
-    hs = _tokens(H, T, 1600)
-    monkeypatch.delenv("WL_BATCHED_SMALL", raising=False)
-    units = _batched(dm, hs)
+    hs = _tokens(H, T, 1600 + T)
+    out = _batched(dm, hs)
     counts = dm.ctx.batched_counts()
-    monkeypatch.setenv("WL_BATCHED_SMALL", "0")
-    grouped = _batched(dm, hs)
-    small = int(((counts >= 1) & (counts <= 8)).sum())
-    print(f"T={T}: {small} experts of 1-8 tokens", flush=True)
-    assert small > 20
-    assert np.array_equal(units.view(np.uint32), grouped.view(np.uint32))
+    print(f"T={T}: {(counts > 0).sum()} experts, at most {counts.max()} tokens, {_small_call(counts, T)}", flush=True)
+    assert _small_call(counts, T) == (single, parts)
+    assert np.array_equal(out, _batched(dm, hs))
+    for t in range(T):
+        assert O.rel_to_scale(_decode(dm, hs[t]), out[t]) < TOL, t
+    src = O.ExpertSource(H, c["moe_inter"], 1)
+    for t in (0, T - 1):
+        assert O.rel_to_scale(O.moe_layer(hs[t], dm.dense[0], src, 0, c)["out"], out[t]) < TOL, t
     dm.close()

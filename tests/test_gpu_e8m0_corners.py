@@ -2,8 +2,8 @@
 
 GLM-shape expert blocks (and the shared expert) with planted rows whose
 scales are the E8M0 corners, so that those values dominate the rows they are
-in, run through the decode kernel (both schedules) and the batched layer (one
-pass of more than 32 tokens per expert), against the oracle's dequant
+in, run through the decode kernel (both schedules) and the batched layer (passes of
+one to four row blocks of 16 tokens per expert), against the oracle's dequant
 (tools/glm_mxfp4_numpy.py:17-26, exact ldexp; src/glm_kernels.cuh:53-61):
 
   gate/up rows (routed SwiGLU values, checked through the mid tap)
@@ -248,36 +248,37 @@ def test_corner_scales_through_decode(corners, shared):
     ctx.set_schedule(moe.SCHED_FUSED)
 
 
+@pytest.mark.parametrize("T", [12, 24, T_BATCH])
 @pytest.mark.parametrize("shared", ["bf16", "mxfp4"])
-def test_corner_scales_through_batched(corners, shared):
+def test_corner_scales_through_batched(corners, shared, T):
+    """Every token goes to the planted experts: a pass of one, two or three row
+    blocks each (one and two: 256 columns a step, scale bytes of their own)."""
     f = corners
     ctx, c = f["ctx"], GLM
     H = c["hidden"]
     sh = _bind_shared(f, shared)
-    hs = f["hs"][3:3 + T_BATCH]
+    hs = f["hs"][3:3 + T]
     d_in = H_.DeviceBuffer.from_array(hs)
-    d_out = H_.DeviceBuffer(4 * H * T_BATCH)
-    ctx.run_moe_batched(0, T_BATCH, d_in.ptr, None, d_out.ptr)
+    d_out = H_.DeviceBuffer(4 * H * T)
+    ctx.run_moe_batched(0, T, d_in.ptr, None, d_out.ptr)
     ctx.check_error()
     counts = ctx.batched_counts()
-    assert counts.max() == T_BATCH  # one pass of 32 tokens and one of 8 per planted expert
-    out = d_out.download(np.float32).reshape(T_BATCH, H)
+    assert counts.max() == T
+    out = d_out.download(np.float32).reshape(T, H)
     ids = None
-    for t in range(T_BATCH):
+    for t in range(T):
         ref = O.moe_layer(hs[t], f["dense"], f["src"], 0, c, shared_f32=sh)
         if ids is None or not np.array_equal(ids, ref["topk_idx"]):
             ids = ref["topk_idx"]
         S, M = _mid_scales(f, ids, O.rms_norm(hs[t], None, c["rms_eps"]))
         _check_rows(f, ids, ref["topk_w"], S[0], M[0], ref["out"], out[t], (shared, "batched", t))
-    print(f"batched ({shared} shared): {T_BATCH} tokens, planted rows within {TOL}", flush=True)
+    print(f"batched ({shared} shared): {T} tokens, planted rows within {TOL}", flush=True)
 
 
 @pytest.mark.parametrize("shared", ["bf16", "mxfp4"])
 def test_corner_scales_through_batched_wide_passes(corners, shared):
     """1024 tokens, all routed to the planted experts: every planted expert
-    (and the shared expert) runs in the batched kernels' wide passes (tokens
-    split evenly over passes of at most 48, the shared expert in passes of
-    64). Twelve tokens spread over the passes are held to the corner bars
+    (and the shared expert) runs in passes of 64 tokens, four row blocks. Twelve tokens spread over the passes are held to the corner bars
     against the oracle; every token's other output rows to 1e-5 against the
     decode kernel (the planted down rows D, E, F scale a SwiGLU value by up to
     2^126, so two implementations that each meet its term-relative bar can

@@ -6,7 +6,7 @@ pass over the threads, and the largest top-k the reference allows
 with 16 shared experts and the weights neither renormalised nor scaled
 (norm_topk_prob false, routed_scaling 1). The decode layer (both schedules)
 against the numpy oracle: ids exact, in order, and every tap and the output
-within 1e-5 rel_to_scale; the batched layer (up to its 816-expert limit)
+within 1e-5 rel_to_scale; the batched layer (up to its 672-expert limit)
 against the decode layer, routing bit for bit (reference router_sigmoid_topk, src/glm_layer_runner.cuh:304-336,
 and run_moe_batched, :818-928)."""
 import numpy as np
@@ -21,6 +21,9 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-5
 SHAPES = [
     dict(hidden=1024, moe_inter=256, n_routed_experts=384, n_experts_per_tok=8, n_shared=1),
+    # the most experts the batched layer takes, and one step more
+    dict(hidden=512, moe_inter=128, n_routed_experts=672, n_experts_per_tok=8, n_shared=1),
+    dict(hidden=512, moe_inter=128, n_routed_experts=688, n_experts_per_tok=8, n_shared=1),
     dict(hidden=768, moe_inter=128, n_routed_experts=1024, n_experts_per_tok=12, n_shared=2),
     dict(hidden=512, moe_inter=128, n_routed_experts=4096, n_experts_per_tok=32, n_shared=1),
     # the widest hidden state, 16 shared experts, weights not renormalised, no scaling
@@ -73,11 +76,11 @@ def test_wide_routing_decode_vs_oracle_and_batched_vs_decode(gpu, shape):
         decoded.append(out)
         routing.append((got["logits"], got["topk_idx"], got["topk_w"]))
     dm.ctx.set_schedule(moe.SCHED_FUSED)
-    # the batched layer over the same tokens (at most 816 experts: its GEMM
+    # the batched layer over the same tokens (at most 672 experts: its GEMM
     # kernels keep the expert tables in LDS; wider configs are refused)
     dh = H_.DeviceBuffer.from_array(hs)
     do = H_.DeviceBuffer(4 * T * H)
-    if c["n_routed_experts"] > 816:
+    if c["n_routed_experts"] > 672:
         with pytest.raises(moe.WindlassError) as ei:
             dm.ctx.run_moe_batched(0, T, dh.ptr, None, do.ptr)
         assert ei.value.status == 1  # WL_ERR_INVALID
