@@ -91,7 +91,7 @@ def test_small_batched_vs_oracle_and_decode(gpu, T):
 
 def test_skewed_routing_multi_pass_and_residual(gpu):
     """A bias that makes the same experts win for every token: those experts
-    get all T tokens (several 32-token passes)."""
+    get all T tokens (two passes, of four and three row blocks of 16)."""
     c = SMALL
     H, E = c["hidden"], c["n_routed_experts"]
     off = np.zeros(E, np.float32)
@@ -136,8 +136,8 @@ def test_glm_batched_64_vs_decode(gpu):
 
 def _oracle_tokens(ids, T, kmt=32, want=10):
     """Tokens to check against the oracle: the first and the last, and tokens
-    of the two experts with the most tokens (more than kmt of them, i.e. run
-    in several passes): the first of each pass boundary and the last."""
+    of the two experts with the most tokens (more than kmt of them, i.e. in passes of
+    three row blocks and more): those on both sides of a row block's end and the last."""
     lists = {}
     for t in range(T):
         for e in ids[t]:
@@ -163,7 +163,7 @@ def test_glm_batched_zipf_vs_decode_and_oracle(gpu, T):
     """Config 3 at the GLM shape with the benchmark's Zipf(1.1) router bias:
     every token's routing equals the decode path's bit for bit and its output
     is within 1e-5 of the decode path's; at least 8 tokens (the first, the
-    last, and tokens on both sides of a 32-token pass boundary of the busiest
+    last, and tokens on both sides of a row block's end of the busiest
     experts) are within 1e-5 of the oracle."""
     c = GLM
     H = c["hidden"]
@@ -191,7 +191,7 @@ def test_glm_batched_zipf_vs_decode_and_oracle(gpu, T):
         assert r < TOL, (t, r)
     pick, multi, hot = _oracle_tokens(ids, T)
     assert len(pick) >= 8
-    assert multi, f"no expert ran more than one 32-token pass at T={T}: {hot}"
+    assert multi, f"no expert of more than 32 tokens at T={T}: {hot}"
     src = O.ExpertSource(H, c["moe_inter"], 15, cache=48)
     worst_ref = 0.0
     for t in pick:

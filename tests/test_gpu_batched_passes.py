@@ -1,7 +1,7 @@
 """The batched layer's passes at their edges on the GPU (run with -m gpu).
 
 An expert's tokens are cut into row blocks of 16 and those into passes of at
-most five (down: four); calls of at most 512 entries group them by expert inside
+most four; calls of at most 2048 entries group them by expert inside
 the gate/up kernel, larger ones in kernels of their own. A bias gives three
 experts every token, so their passes end at, before and after a block and a
 pass; the other three choices spread thinly over the rest. Every token is
@@ -45,12 +45,12 @@ def test_passes_at_block_edges(gpu, T, shape):
     dm.close()
 
 
-@pytest.mark.parametrize("E,K,T", [(48, 1, 512), (48, 1, 513), (624, 1, 512), (640, 1, 512), (48, 8, 64), (16, 16, 32),
-                                   (624, 2, 31)])
+@pytest.mark.parametrize("E,K,T", [(48, 1, 512), (48, 1, 513), (48, 1, 2048), (48, 1, 2049), (192, 1, 2048), (208, 1, 2048),
+                                   (624, 1, 512), (640, 1, 512), (48, 8, 64), (48, 8, 256), (16, 16, 32), (624, 2, 31)])
 def test_entries_grouped_by_expert(gpu, E, K, T):
-    """Up to 512 entries are grouped inside the gate/up kernel (a bit per token and
-    expert; up to 624 experts), more of them, or more experts, by kernels of their
-    own. Hidden 256 and inter 128: a unit is one step. Counts equal the ids'; every
+    """Up to 2048 entries are grouped inside the gate/up kernel (one to four a thread;
+    a bit per token and expert, 48 KB of them), more of them, more bits, or more
+    experts than leave room for the tokens, by kernels of their own. Hidden 256 and inter 128: a unit is one step. Counts equal the ids'; every
     seventh token and the last agree with the decode path."""
     c = dict(SMALL, hidden=256, moe_inter=128, n_routed_experts=E, n_experts_per_tok=K)
     dm = DeviceModel(c, seed=22, n_layers=1)

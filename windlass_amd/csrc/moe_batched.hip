@@ -1,36 +1,37 @@
 // moe_batched.hip — the MoE layer for T tokens at once on gfx950 (the
 // reference's run_moe_batched, src/glm_layer_runner.cuh:818-928, used by
-// prefill): every expert's weights are streamed once per pass of up to kMT of
-// its tokens instead of once per token.
+// prefill): an expert's weights are read once per pass of up to 64 of its tokens
+// instead of once per token.
 //
-//   bnorm    RMSNorm per token -> norm (f32, for the router) and norm3 (the
-//            three bf16 pieces the GEMMs read)
+//   bnorm    RMSNorm per token -> norm (f32) and, for a bf16 shared expert, norm3
+//            (its three bf16 pieces)
 //   broute   router logits, kTB tokens per work-group; norm and logits use the
 //            arithmetic of the decode and routing kernels, so a token's ids
 //            equal the ones wl_run_moe selects for it
-//   btopk    sigmoid + bias, top-k, weights (one work-group per token)
+//   btopk    sigmoid + bias, top-k, weights (one work-group per token), and the
+//            token's row of norm quantised in place (q6.h)
 //   bcount   per expert: its entries (token*K + slot) in ascending order
 //            (wave ballots, deterministic) and their count
 //   bscatter per expert: its compact range (prefix of the counts), ent/pos
-//   bup      gate/up + SwiGLU: shared expert (unit = token pass x 64 rows),
-//            routed experts (unit = expert pass x 4 x 64 rows); a routed
-//            pass's activation DMAs read its tokens' norm3 rows in place,
-//            through a per-work-group table of its units' tokens in LDS, so
-//            no expert-major copy of the activations is made
-//   bdown    down: shared expert (unit = token pass x 128 rows), routed
-//            experts (unit = expert pass x 512 rows)
+//            (calls of few entries: both inside bup, group_entries)
+//   bup      gate/up + SwiGLU: shared expert (unit = token pass x 64 or 128 rows),
+//            routed experts (unit = expert pass x 4 x 64 rows) -> midf, compact
+//            rows; a routed pass's activation DMAs read its tokens' quantised rows
+//            in place, through tables of tokens in LDS
+//   bquant   the rows of midf quantised -> mid6
+//   bdown    down: shared expert (unit = token pass x 128 or 256 rows), routed
+//            experts (unit = expert pass x 512 rows) -> expout
 //   bcomb    out[t] = (resid[t] +) sum_k w[t][k] e_k[t] (slot order) + shared[t]
 //
-// The GEMMs run each activation as three bf16 pieces (x = p0 + p1 + p2 to f32
-// precision) through v_mfma_f32_16x16x32_bf16; MXFP4 weights are converted
-// exactly to bf16 (v_cvt_scalef32_pk_bf16_fp4), bf16 weights are used as they
-// are. bup and bdown are persistent (one work-group per CU) and share one step
-// pipeline: activations arrive in LDS by DMA, weights two steps ahead in
-// registers.
+// The routed GEMMs run each activation as 6-bit pieces against the MXFP4 weights as
+// they are on the scaled matrix instruction (q6.h), the bf16 shared expert's as three
+// bf16 pieces (x = p0 + p1 + p2 to f32 precision) through v_mfma_f32_16x16x32_bf16.
+// bup and bdown are persistent (one work-group per CU) and share one step pipeline
+// (batched_gemm.h): activations arrive in LDS by DMA, weights two steps ahead in
+// registers. A dense layer of many positions has kernels of its own (batched_dense.h).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cstdlib>
 #include <type_traits>
 
 #include "dev_common.h"
@@ -462,11 +463,12 @@ WL_DEV Pass pass_at(const PassTab& pt, uint32_t E, uint32_t j) {
 }
 
 // ---- token table -------------------------------------------------------------
-// A routed pass's activations are its tokens' rows of norm3, read in place by
+// A routed pass's activations are its tokens' quantised rows of norm, read in place by
 // the DMAs. Before a gate/up pipeline runs, its work-group writes the tokens
 // of its units' passes into LDS, tt[W i + m] = the token of row m of its unit
 // i (W: the pipeline's largest pass), in one round of global loads for the
-// whole pipeline; a unit's bind then reads its lane's two tokens there. (A
+// whole pipeline; a unit's bind then reads its lanes' tokens there. (A call whose
+// entries bup groups itself has the tokens of all entries there instead.) (A
 // prefetch into registers would cost a wait at every bind: the compiler does
 // not know how many steps lie between a load and its use.) The host sizes
 // the table (BatchArgs::tcap entries) for the most units a work-group can
