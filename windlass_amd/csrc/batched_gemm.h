@@ -432,7 +432,7 @@ WL_DEV void pair_swap(u32x4& x, u32x4& y) {
 // land as zeros (zero scales too: their products are zero).
 template <uint32_t MB>
 struct AStreamQ {
-    rsrc_t rs;
+    rsrc_t rs, rs1;  // (rs1: of further pieces beside the records)
     // lane byte offsets of the lane's units of its rows (left: of its left-over
     // unit), k tiles of a row, bytes of a record
     uint32_t base[MB], left, nk, rec;
@@ -444,11 +444,13 @@ struct AStreamQ {
 // is four slices, or 16 row pairs: four tiles per wave (tile 8 sl + v of slice
 // sl, row pairs 2 v and 2 v + 1 of the 16), as the native block's batched scale
 // words are laid out. NB row blocks, KT k tiles per step.
-template <bool UP, uint32_t NB, uint32_t KT>
+// FOLD (NB = 1): a row's further pieces stand beside its record, as a second row block.
+template <bool UP, uint32_t NB, uint32_t KT, bool FOLD = false>
 struct QBase {
-    using AS = AStreamQ<NB>;
+    static constexpr uint32_t MB = FOLD ? 2u : NB;  // row blocks staged
+    using AS = AStreamQ<MB>;
     static constexpr uint32_t P = kQP, NG = (kQUnits + 3u) / 4u;  // groups of a record
-    static constexpr uint32_t kTiles = NB * KT, kTileB = 1024u * NG, kDmas = kTiles + 1u;
+    static constexpr uint32_t kTiles = MB * KT, kTileB = 1024u * NG, kDmas = kTiles + 1u;
     static_assert(NG == 10u && kTiles <= 4u, "ten groups of at most four tiles");
     static_assert(kTileB * kTiles + 8192u <= kSlotB, "a step's tiles fit a slot");
     const DecodeArgs& a;
@@ -498,7 +500,7 @@ struct QBase {
     // A unit with a row of further pieces runs its steps twice: on the records, then
     // on the further pieces.
     WL_MEM bool twice(const UnitInfo& x, uint32_t i) const {
-        if (!any || !x.live) return false;
+        if (FOLD || !any || !x.live) return false;
         static_assert(kRB * NB <= 64u, "a lane per row");
         const bool has = lane < x.nt && gld((UP ? b.more_up : b.more_dn) + row_of(x, i, min(lane, x.nt - 1u))) != 0u;
         return __builtin_amdgcn_ballot_w64(has) != 0u;
@@ -523,36 +525,39 @@ struct QBase {
         const uint32_t kd = UP ? H : I, n = 8u * (v & 1u) + lane / 8u, c8 = lane % 8u ^ q_swizzle(n);
         const uint32_t nrow = UP ? b.T : b.T * (K + ((b.flags & kBatchShared4) ? 1u : 0u));
         const uint32_t rec = (uint32_t)q6_row_bytes(kd), ext = (uint32_t)q6_more_bytes(kd);
-        const uint32_t rowb = UP ? rec + ext : more ? ext : rec, row0 = UP && more ? rec : 0u;
-        const uint8_t* rows = UP ? (const uint8_t*)b.norm : more ? b.mid6x : b.mid6;
-        A.rs = make_rsrc(x.live ? rows : nullptr, x.live ? nrow * rowb : 0u);
+        auto array = [&](bool lo) {
+            const uint8_t* rows = UP ? (const uint8_t*)b.norm : lo ? b.mid6x : b.mid6;
+            return make_rsrc(x.live ? rows : nullptr, x.live ? nrow * (UP ? rec + ext : lo ? ext : rec) : 0u);
+        };
+        A.rs = array(more);
+        if (FOLD) A.rs1 = array(true);
         A.nk = x.live ? nk : 0u;
         A.rec = more ? kQMore : kQRecord;
-        // the lane's unit c of row m's record
+        // the lane's unit c of its row of block m
         auto row_at = [&](uint32_t m, uint32_t c) {
-            const uint32_t r = kRB * m + n;
+            const bool lo = more || (FOLD && m == 1u);
+            const uint32_t r = FOLD ? n : kRB * m + n;
             const uint32_t row = x.live ? row_of(x, i, r) : 0u;
             bool has = r < x.nt && c < kQUnits;
-            if (more) {
+            if (lo) {
                 has = has && gld((UP ? b.more_up : b.more_dn) + row) != 0u && q6_more_unit(c) != ~0u;
                 c = q6_more_unit(c);
             }
-            return has ? row * rowb + row0 + 16u * c : kOOBV;
+            return has ? row * (UP ? rec + ext : lo ? ext : rec) + (UP && lo ? rec : 0u) + 16u * c : kOOBV;
         };
 #pragma unroll
-        for (uint32_t m = 0; m < NB; m++) A.base[m] = row_at(m, 8u * (v / 2u) + c8);
-        A.left = v / 2u < kTiles ? row_at(v / 2u % NB, 32u + c8) : kOOBV;
+        for (uint32_t m = 0; m < MB; m++) A.base[m] = row_at(m, 8u * (v / 2u) + c8);
+        A.left = v / 2u < kTiles ? row_at(v / 2u % MB, 32u + c8) : kOOBV;
     }
     template <int SL>
     WL_MEM void dma(const AS& A, uint32_t s, uint32_t j) const {
-        if (j < kTiles) {
-            const uint32_t k = s * KT + j / NB;
-            dma16<SL>(A.rs, j * kTileB + v * 1024u, k < A.nk ? A.base[j % NB] : kOOBV, k * A.rec);
-        } else {
-            const uint32_t t = v / 2u, k = s * KT + t / NB;
-            dma16<SL>(A.rs, t < kTiles ? t * kTileB + (8u + v % 2u) * 1024u : kTiles * kTileB + v * 1024u,
-                      k < A.nk ? A.left : kOOBV, k * A.rec);
-        }
+        // (wave v's left-over units are those of tile v / 2)
+        const uint32_t t = j < kTiles ? j : v / 2u, k = s * KT + t / MB;
+        const bool lo = FOLD && t % MB == 1u;
+        const uint32_t dst = j < kTiles ? j * kTileB + v * 1024u
+                             : t < kTiles ? t * kTileB + (8u + v % 2u) * 1024u : kTiles * kTileB + v * 1024u;
+        dma16<SL>(lo ? A.rs1 : A.rs, dst, k >= A.nk ? kOOBV : j < kTiles ? A.base[j % MB] : A.left,
+                  k * (lo ? kQMore : A.rec));
     }
     WL_MEM bool unit_end() {
         csecond = ctwice && !csecond;
@@ -596,11 +601,14 @@ struct QBase {
 // 4 slices x 2 k tiles; down: 4 slices of 64 columns x 2 row pairs. The first piece and the
 // others sum in accumulators of their own; in passes of one row block the first
 // piece's are added to the sums at every step in f32 (matrix instructions that
-// add into a large sum round it more coarsely).
-template <bool UP, uint32_t NB>
-struct QNarrow : QBase<UP, NB, 2> {
-    using QB = QBase<UP, NB, 2>;
+// add into a large sum round it more coarsely). With FOLD a call with further pieces
+// reads the weights of its small passes once (a second run of their steps: 7 and 64 tokens with
+// outliers in every one 299 and 832 us); a pass without them gives the same bits.
+template <bool UP, uint32_t NB, bool FOLD = false>
+struct QNarrow : QBase<UP, NB, 2, FOLD> {
+    using QB = QBase<UP, NB, 2, FOLD>;
     using QB::P;
+    using QB::MB;
     struct WB {
         u32x4 w[8];
         uint32_t s[2];
@@ -629,28 +637,28 @@ struct QNarrow : QBase<UP, NB, 2> {
             if (kSum) sum[t] = z;
         }
     }
-    // Operands it = (P q + p) NB + m in this order; each runs against the wave's
+    // Operands it in this order: piece p of block m of k tile q, it = (P q + p) NB + m
+    // (FOLD: after a k tile's six pieces its further ones); each runs against the wave's
     // weight tiles while the two after it are read.
     template <class Next>
     WL_MEM void comp(uint32_t, const uint8_t* sl, WB& W, Next next) {
-        constexpr uint32_t N = 2u * P * NB, AH = 2u;
+        constexpr uint32_t NQ = FOLD ? P + kQX : P * NB, N = 2u * NQ, AH = 2u;
         i32x8 af[AH + 1u];
-        u32x2 sa[NB];
+        u32x2 sa[MB];
         uint32_t sx = 0u, sy = 0u;
         const uint32_t lo16 = this->lo16;
-        auto tile = [&](uint32_t q, uint32_t m) { return sl + (q * NB + m) * QB::kTileB; };
-        auto frag = [&](uint32_t it) {
-            const uint32_t m = it % NB, p = it / NB % P, q = it / (NB * P);
-            return q_frag(tile(q, m), p, lo16, this->lo8);
-        };
+        auto tile = [&](uint32_t q, uint32_t m) { return sl + (q * MB + m) * QB::kTileB; };
+        auto block = [](uint32_t it) { return FOLD ? (it % NQ >= P ? 1u : 0u) : it % NB; };
+        auto piece = [](uint32_t it) { return FOLD ? (it % NQ >= P ? it % NQ - P : it % NQ) : it / NB % P; };
+        auto frag = [&](uint32_t it) { return q_frag(tile(it / NQ, block(it)), piece(it), lo16, this->lo8); };
 #pragma unroll
         for (uint32_t it = 0; it < AH; it++) af[it] = frag(it);
 #pragma unroll
         for (uint32_t it = 0; it < N; it++) {
-            const uint32_t m = it % NB, p = it / NB % P, q = it / (NB * P);
-            if (p == 0u && m == 0u) {
+            const uint32_t m = block(it), p = piece(it), q = it / NQ;
+            if (it % NQ == 0u) {
 #pragma unroll
-                for (uint32_t i = 0; i < NB; i++) sa[i] = q_scales(tile(q, i), this->lo8);
+                for (uint32_t i = 0; i < MB; i++) sa[i] = q_scales(tile(q, i), this->lo8);
                 if (!UP) {
 #pragma unroll
                     for (uint32_t h = 0; h < 2; h++) pair_swap(W.w[4u * q + h], W.w[4u * q + 2u + h]);
@@ -666,8 +674,9 @@ struct QNarrow : QBase<UP, NB, 2> {
                 const uint32_t sw = UP ? W.s[t >> 1] : (t & 2u) ? sy : sx;
                 const u32x4 w = W.w[UP ? 2u * t + q : 4u * q + t];
                 const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-                f32x4& c = acc[t][m][p == 0u ? 0u : 1u];
-                c = mmq(w, af[it % (AH + 1u)], kSum && p == 0u && q == 0u ? z : c, ow, sw, p & 3u, p < 4u ? sa[m].x : sa[m].y);
+                const bool first = p == 0u && !(FOLD && m == 1u);
+                f32x4& c = acc[t][FOLD ? 0u : m][first ? 0u : 1u];
+                c = mmq(w, af[it % (AH + 1u)], kSum && first && q == 0u ? z : c, ow, sw, p & 3u, p < 4u ? sa[m].x : sa[m].y);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -896,10 +905,10 @@ WL_DEV ExpertTab load_expert_tab(const BatchArgs& b, uint32_t E, uint32_t K, uin
     return et;
 }
 // The routed passes of NB row blocks at pl; returns their units' count.
-template <bool UP, uint32_t NB>
+template <bool UP, uint32_t NB, bool FOLD = false>
 WL_DEV uint32_t run_routed(const DecodeArgs& a, const BatchArgs& b, uint32_t E, const ExpertTab& et,
                            const uint8_t* const* stab, Places pl, bool any, bool single) {
-    using Kn = std::conditional_t<(NB > 2u), QWide<UP, NB>, QNarrow<UP, NB>>;
+    using Kn = std::conditional_t<(NB > 2u), QWide<UP, NB>, QNarrow<UP, NB, FOLD>>;
     const PassTab pt = load_pass_tab(et, E, NB, single);
     pipeline_drain();
     const uint32_t H = a.H, I = a.I;
@@ -996,5 +1005,8 @@ WL_DEV void run_gemm(const DecodeArgs* pa, const BatchArgs& b) {
     if (sizes & 1u << 4) u += run_routed<UP, 4>(a, b, E, et, stab, Places::from(u, skip), any, single);
     if (sizes & 1u << 3) u += run_routed<UP, 3>(a, b, E, et, stab, Places::from(u, skip), any, single);
     if (sizes & 1u << 2) u += run_routed<UP, 2>(a, b, E, et, stab, Places::from(u, skip), any, single);
-    if (sizes & 1u << 1) run_routed<UP, 1>(a, b, E, et, stab, Places::from(u, skip), any, single);
+    if (sizes & 1u << 1) {
+        if (any) run_routed<UP, 1, true>(a, b, E, et, stab, Places::from(u, skip), any, single);
+        else run_routed<UP, 1>(a, b, E, et, stab, Places::from(u, skip), any, single);
+    }
 }
