@@ -251,8 +251,9 @@ wl_status wl_run_chain(wl_ctx* ctx, uint32_t first_layer, uint32_t n_layers, flo
  * grouped by expert (stable, (token, slot) order) and every selected expert's
  * weights are read once per pass of up to 64 of its tokens; the per-token combine sums
  * the slots in slot order, then the shared expert (the reference's pass 3). The
- * inputs and SwiGLU values of MXFP4 experts keep f32 precision wherever a value is
- * at least 2^-15 of the largest of its 32 neighbours and 2^-105 itself.
+ * inputs and SwiGLU values of MXFP4 experts are held to 2^-29 of the largest of the
+ * 32 that share a weight scale, or to 2^-39 in rows where the former might show in
+ * sums that leave out the few largest; no finer than 2^-129.
  * A layer with every expert bound runs with no host round trip; a layer with
  * none bound fetches its routed set through the context's expert source (see
  * wl_expert_source: one host round trip per chunk of tokens, each unique

@@ -75,6 +75,7 @@ struct DenseK {
     UnitInfo cu;  // e: its split
     f32x4 acc[2][NB], sum[2][NB], err[2][NB];
 
+    static constexpr bool kOnce = true;
     WL_MEM static bool unit_end() { return true; }
     WL_MEM UnitInfo unit(uint32_t i) const {
         UnitInfo x{false, 0u, 0u, 0u, 0u};

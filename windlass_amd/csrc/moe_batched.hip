@@ -62,11 +62,15 @@ WL_DEV void split3_any(float x, uint32_t& h, uint32_t& m, uint32_t& l) {
 // (ANY: of values that may leave bf16's range).
 template <bool ANY = false>
 WL_DEV void store_pieces4(uint16_t* p, uint32_t stride, const float (&x)[4]) {
-    uint32_t h[4], md[4], l[4];
+    uint32_t h[4], md[4], l[4], mx = 0u;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-        if constexpr (ANY) split3_any(x[q], h[q], md[q], l[q]);
-        else split3(x[q], h[q], md[q], l[q]);
+        split3(x[q], h[q], md[q], l[q]);
+        mx = max(mx, __float_as_uint(x[q]) & 0x7FFFFFFFu);
+    }
+    if (ANY && mx >= 0x7F7F8000u) {  // (rounds to infinity)
+#pragma unroll
+        for (int q = 0; q < 4; q++) split3_any(x[q], h[q], md[q], l[q]);
     }
     auto pack = [](const uint32_t (&x)[4]) {
         return (uint64_t)(x[0] | (x[1] << 16)) | ((uint64_t)(x[2] | (x[3] << 16)) << 32);

@@ -16,19 +16,19 @@
 // a few, as beside the outlier channels of a trained model, weights that are zero at
 // those few (MXFP4 rounds many to zero) leave a sum of the small ones alone; with five
 // pieces such sums were off by 3e-6 of the largest output at 100 times, 1e-3 at 30000
-// times, and six leave a 32nd of that. A row in which this may count therefore has two
-// further pieces per block, in records of their own that the GEMMs run against the
-// same weights, into the same sums: 2^-39 of the largest value, full
-// f32 precision down to 1/32768 of it. It counts where what six pieces leave of the
+// times, and six leave a 32nd of that. A row in which this may count therefore has
+// two further pieces per block, in records of their own that the GEMMs run against
+// the same weights, into the same sums: 2^-39 of the largest value, full f32
+// precision down to 1/32768 of it. It may count where what six pieces leave of the
 // wide blocks, some 2^-31 of the largest for each of 32 values, may exceed 2^-24.5 of
-// the row's sum without their few large values (q6_more). The row's other blocks are in
-// that sum: SwiGLU values of large gate values, half of them almost zero, make many
-// blocks wide and lose nothing (a rule block by block took further pieces for them and
-// 64 tokens 755 to 940 us). Passes of such rows of at most 16 tokens
-// have them beside the records, larger ones run twice as long (hidden 6144, inter 2048,
-// 8 of 256 experts, 12 columns 1000 times the rest in every token, with three bf16
-// pieces and now: 7 tokens 208 and 209 us, 64 563 and 553, 256 1012 and 1030, 1000 2345 and
-// 2187, 4096 8152 and 7238).
+// the row's sum without their few large values (q6_more). The row's other blocks are
+// in that sum: SwiGLU values of large gate values, half of them almost zero, make many
+// blocks wide and lose nothing (a rule block by block took further pieces for them,
+// and 64 tokens 755 to 940 us). Passes of such rows of at most 16 tokens have them
+// beside the records, larger ones run twice as long (hidden 6144, inter 2048, 8 of 256
+// experts, 12 columns 1000 times the rest in every token, with three bf16 pieces and
+// now: 7 tokens 208 and 209 us, 64 563 and 553, 256 1012 and 1030, 1000 2345 and 2187,
+// 4096 8152 and 7238).
 //
 // Why this format: measured on MI355X the instruction runs 8.5 PFLOP/s with 6-bit
 // against 4-bit operands (bf16 2.43, 8-bit 4.8), so six pieces cost 0.6 of three
