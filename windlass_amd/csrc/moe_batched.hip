@@ -269,13 +269,11 @@ __global__ void __launch_bounds__(kThreads) btopk_kernel(const DecodeArgs* __res
         topk_score(gld(b.logits + (size_t)t * E + e), gld(a.bias + e), e, tk_sc, tk_ch);
     lds_barrier();  // (every thread's reads of the row are done)
     f32x16 even, odd;
-    QRange rg{0.0, 0.0, false};
     auto quantise = [&](uint32_t i) {
         if (i >= H / 32u) return;
         q6_load(row + 36u * i, even, odd);
         const uint32_t mx = q6_max(even, odd);
-        rg = q6_range(even, odd, mx);
-        if (rg.wide) wide = 1u;
+        if (q6_wide(even, odd, mx)) wide = 1u;
         q6_store<false>((uint8_t*)rowp + (i / 4u) * kQRecord, i % 4u, even, odd, mx);
     };
     // up to 256 experts the argmax is wave 0's: the other waves quantise (at most
@@ -294,6 +292,11 @@ __global__ void __launch_bounds__(kThreads) btopk_kernel(const DecodeArgs* __res
     }
     bool more = false;
     if (wide != 0u) {
+        QRange rg{0.0, 0.0};
+        if (tid < H / 32u) {
+            q6_load(row + 36u * tid, even, odd);
+            rg = q6_range(even, odd);
+        }
         const double big = wave_sum_f64(rg.big), rest = wave_sum_f64(rg.rest);
         if ((tid & 63u) == 0u) {
             part[0][tid >> 6] = big;
@@ -579,7 +582,6 @@ __global__ void __launch_bounds__(256) bquant_kernel(const DecodeArgs* __restric
     const float* mid = b.midf + (size_t)row * b.ldm;
     f32x16 even, odd;
     bool wide = false;
-    double big = 0.0, rest = 0.0;
     for (uint32_t b0 = 0; b0 < nb; b0 += 64u) {
 #pragma unroll
         for (uint32_t i = 0; i < 8; i++) {
@@ -591,16 +593,22 @@ __global__ void __launch_bounds__(256) bquant_kernel(const DecodeArgs* __restric
         if (live && k < nb) {
             q6_load(xs[v] + 36u * lane, even, odd);
             const uint32_t mx = q6_max(even, odd);
-            const QRange rg = q6_range(even, odd, mx);
-            wide |= rg.wide;
-            big += rg.big;
-            rest += rg.rest;
+            wide |= q6_wide(even, odd, mx);
             q6_store<false>(b.mid6 + (size_t)row * q6_row_bytes(I) + (k / 4u) * kQRecord, k % 4u, even, odd, mx);
         }
         lds_barrier();
     }
     bool more = false;
-    if (__builtin_amdgcn_ballot_w64(wide) != 0u) more = q6_more(wave_sum_f64(big), wave_sum_f64(rest));
+    if (__builtin_amdgcn_ballot_w64(wide) != 0u) {
+        double big = 0.0, rest = 0.0;
+        for (uint32_t k = lane; k < nb; k += 64u) {
+            q6_load(mid + 32u * k, even, odd);
+            const QRange rg = q6_range(even, odd);
+            big += rg.big;
+            rest += rg.rest;
+        }
+        more = q6_more(wave_sum_f64(big), wave_sum_f64(rest));
+    }
     if (live && lane == 0u) {
         gst(b.more_dn + row, more ? 1u : 0u);
         if (more) gst(b.more + 1, 1u);

@@ -81,34 +81,43 @@ WL_DEV uint32_t q6_max(const f32x16& even, const f32x16& odd) {
     }
     return mx;
 }
-// What a block of largest magnitude mx adds to its row's test for further pieces
-// (q6_more). big: the square of the largest value if the block is wide, that is at most
-// eight of its values are within 2^8 of the largest and smaller ones are there. rest:
-// the sum of squares of those smaller ones; in other blocks that of the values under an
-// eighth of the largest, if at most eight reach that (outliers, too), or of all.
+// Whether a block of largest magnitude mx is wide: at most eight of its values are
+// within 2^8 of the largest, and smaller ones are there.
+WL_DEV bool q6_wide(const f32x16& even, const f32x16& odd, uint32_t mx) {
+    const float m = __uint_as_float(mx), lim = m * 0x1p-8f;
+    uint32_t n = 0u, zero = 0u;
+#pragma unroll
+    for (int i = 0; i < 16; i++) n += (fabsf(even[i]) >= lim ? 1u : 0u) + (fabsf(odd[i]) >= lim ? 1u : 0u);
+    if (n > 8u || m < 0x1p-100f || !(m < INFINITY)) return false;
+#pragma unroll
+    for (int i = 0; i < 16; i++) zero += (even[i] == 0.f ? 1u : 0u) + (odd[i] == 0.f ? 1u : 0u);
+    return n + zero < 32u;
+}
+// What a block adds to the test of a row with wide blocks (q6_more). big: the square
+// of the largest value if the block is wide. rest: the sum of squares of the smaller
+// ones; in other blocks that of the values under an eighth of the largest, if at most
+// eight reach that (outliers, too), or of all.
 struct QRange {
     double big, rest;
-    bool wide;
 };
-WL_DEV QRange q6_range(const f32x16& even, const f32x16& odd, uint32_t mx) {
+WL_DEV QRange q6_range(const f32x16& even, const f32x16& odd) {
+    const uint32_t mx = q6_max(even, odd);
     const float m = __uint_as_float(mx), inv = __builtin_amdgcn_rcpf(m);
+    if (m < 0x1p-100f || !(m < INFINITY)) return QRange{0.0, 0.0};
+    const bool wide = q6_wide(even, odd, mx);
     float all = 0.f, s3 = 0.f, s8 = 0.f;
-    uint32_t n3 = 0u, n8 = 0u, zero = 0u;
+    uint32_t n3 = 0u;
 #pragma unroll
     for (int i = 0; i < 32; i++) {
-        const float a = fabsf(i & 1 ? odd[i / 2] : even[i / 2]) * inv, q = a * a;
-        const bool l3 = a >= 0x1p-3f, l8 = a >= 0x1p-8f;
+        const float v = fabsf(i & 1 ? odd[i / 2] : even[i / 2]), a = v * inv, q = a * a;
+        const bool l3 = a >= 0x1p-3f;
         all += q;
         s3 += l3 ? 0.f : q;
-        s8 += l8 ? 0.f : q;
+        s8 += v >= m * 0x1p-8f ? 0.f : q;
         n3 += l3 ? 1u : 0u;
-        n8 += l8 ? 1u : 0u;
-        zero += a == 0.f ? 1u : 0u;
     }
-    if (m < 0x1p-100f || !(m < INFINITY)) return QRange{0.0, 0.0, false};
-    const bool wide = n8 <= 8u && n8 + zero < 32u;
     const double m2 = (double)m * (double)m;
-    return QRange{wide ? m2 : 0.0, m2 * (wide ? s8 : n3 <= 8u ? s3 : all), wide};
+    return QRange{wide ? m2 : 0.0, m2 * (wide ? s8 : n3 <= 8u ? s3 : all)};
 }
 // From the row's sums.
 WL_DEV bool q6_more(double big, double rest) { return big > 256.0 * rest; }
