@@ -922,8 +922,8 @@ def main():
         "dtype": ("mxfp4/bf16 weights, f32 activations and accumulation (bf16 MFMA on three exact bf16 pieces "
                   "of each f32 activation); the cross-work-group partial sums are exchanged as f32 rounded to "
                   "21 stored mantissa bits" if not batched else
-                  "mxfp4/bf16 weights, f32 activations and accumulation (scaled MFMA on five or six fp6 pieces of each "
-                  "f32 activation against the fp4 weights, bf16 MFMA on three bf16 pieces against the bf16 ones)"),
+                  "mxfp4/bf16 weights, f32 activations and accumulation (scaled MFMA on six fp6 pieces of each f32 "
+                  "activation, eight beside outliers, against the fp4 weights, bf16 MFMA on three bf16 pieces against the bf16 ones)"),
         "data": "synthetic",
         "config": {"workload": (f"config3: one GLM MoE layer over {args.tokens} tokens (batched"
                                 f"{', allocation-free entry point' if args.noalloc else ''})" if batched else

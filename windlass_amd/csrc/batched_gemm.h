@@ -970,10 +970,10 @@ WL_DEV uint32_t run_routed(const DecodeArgs& a, const BatchArgs& b, uint32_t E, 
 // Routed rows as fp6 pieces against fp4 weights run at 3.5 times the rate of bf16
 // pieces and need no conversion of the weights. Whole calls, hidden 6144, inter
 // 2048, 8 of 256 experts (256 work-groups of eight waves), before (bf16 pieces,
-// passes of 32 and 64) and now: 4096 tokens 8360 and 5180 us, 1000 tokens 2307 and
-// 1601, 64 tokens (one row block per expert; the weights' 4.4 GB at 6 TB/s) 751 and
-// 757, 7 tokens 215.7 and 218.1; hidden 2944, inter 1408, 6 of 160 experts, 333 tokens: 462 and 305.
-// Error against 64 bits: 8.1e-7 and 4.5e-7 at 4096 tokens, 3.5e-7 and 1.5e-7 at 64.
+// passes of 32 and 64) and now: 4096 tokens 8435 and 5165 us, 1000 tokens 2309 and
+// 1594, 64 tokens (one row block per expert; the weights' 4.4 GB at 6.2 TB/s) 735 and
+// 732, 7 tokens 209 and 205; hidden 2944, inter 1408, 6 of 160 experts, 333 tokens: 465 and 313.
+// Error against 64 bits: 8.1e-7 and 4.6e-7 at 4096 tokens, 3.6e-7 and 1.5e-7 at 64.
 template <bool UP>
 WL_DEV void run_gemm(const DecodeArgs* pa, const BatchArgs& b) {
     const DecodeArgs& a = *pa;
