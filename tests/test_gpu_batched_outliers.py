@@ -54,8 +54,9 @@ def _wide(b):
 
 
 def _ffn(x, w):
-    g = x @ w[0].T
-    return (g / (1.0 + np.exp(-g)) * (x @ w[1].T)) @ w[2].T
+    g = x @ w[0].T  # (exp may overflow: the value is 0 then)
+    with np.errstate(over="ignore"):
+        return (g / (1.0 + np.exp(-g)) * (x @ w[1].T)) @ w[2].T
 
 
 @pytest.mark.parametrize("ratio", [1, 100, 2000, 30000])
